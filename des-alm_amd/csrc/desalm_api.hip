@@ -58,9 +58,8 @@ struct WarmStart {
     float* stats = nullptr;  // kWsStats: feature mu, 1/sd (kWsIn each), target scale (kWsComp), unused
     bool have_stats = false;
     int bcap = 0;  // rows of the scratch matrices
-    float *A0 = nullptr, *A1 = nullptr, *A2 = nullptr, *Y = nullptr, *Tb = nullptr;
-    float *dZ3 = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *P = nullptr;
-    double* lpart = nullptr;  // loss partial sums, kWsLossParts per training iteration
+    MlpBuf b{};
+    double* loss = nullptr;  // loss sum per training iteration
     long lcap = 0;
     std::vector<void*> dev;
     long long bytes = 0;
@@ -68,7 +67,6 @@ struct WarmStart {
     int o2() const { return (kWsIn + 1) * nh; }
     int o3() const { return (kWsIn + 1) * nh + (nh + 1) * nh; }
 };
-constexpr int kWsLossParts = 64;
 
 struct desalm_ctx {
     desalm_params p;
@@ -611,39 +609,30 @@ int ws_scratch(desalm_ctx* c, int m) {
     WarmStart& w = c->ws;
     if (m <= w.bcap) return 0;
     const int nh = w.nh;
-    w.A0 = ws_alloc<float>(c, (long)m * (kWsIn + 1));
-    w.A1 = ws_alloc<float>(c, (long)m * (nh + 1));
-    w.A2 = ws_alloc<float>(c, (long)m * (nh + 1));
-    w.Y = ws_alloc<float>(c, (long)m * kWsOut);
-    w.Tb = ws_alloc<float>(c, (long)m * kWsTgt);
-    w.dZ3 = ws_alloc<float>(c, (long)m * kWsOut);
-    w.dZ2 = ws_alloc<float>(c, (long)m * nh);
-    w.dZ1 = ws_alloc<float>(c, (long)m * nh);
-    w.P = ws_alloc<float>(c, (long)wgrad_parts(m) * (kWsIn + 1) * nh);
-    if (!w.A0 || !w.A1 || !w.A2 || !w.Y || !w.Tb || !w.dZ3 || !w.dZ2 || !w.dZ1 || !w.P) return -1;
+    MlpBuf& b = w.b;
+    b.A0 = ws_alloc<float>(c, (long)m * (kWsIn + 1));
+    b.A1 = ws_alloc<float>(c, (long)m * (nh + 1));
+    b.A2 = ws_alloc<float>(c, (long)m * (nh + 1));
+    b.Y = ws_alloc<float>(c, (long)m * kWsOut);
+    b.Tb = ws_alloc<float>(c, (long)m * kWsTgt);
+    b.dZ3 = ws_alloc<float>(c, (long)m * kWsOut);
+    b.dZ2 = ws_alloc<float>(c, (long)m * nh);
+    b.dZ1 = ws_alloc<float>(c, (long)m * nh);
+    b.P = ws_alloc<float>(c, (long)wgrad_parts(m) * w.np());
+    b.lpart = ws_alloc<double>(c, mlp_tiles(m));
+    if (!b.A0 || !b.A1 || !b.A2 || !b.Y || !b.Tb || !b.dZ3 || !b.dZ2 || !b.dZ1 || !b.P || !b.lpart) return -1;
     w.bcap = m;
     return 0;
 }
 
-// forward pass of m rows already in A0
-void ws_forward(desalm_ctx* c, hipStream_t s, int m) {
+// room for the loss sums of n training iterations (grown, never shrunk)
+int ws_losses(desalm_ctx* c, long n) {
     WarmStart& w = c->ws;
-    const int nh = w.nh;
-    launch_dense(s, w.A0, kWsIn + 1, kWsIn + 1, w.w, nh, w.A1, nh + 1, m, 1, 1);
-    launch_dense(s, w.A1, nh + 1, nh + 1, w.w + w.o2(), nh, w.A2, nh + 1, m, 1, 1);
-    launch_dense(s, w.A2, nh + 1, nh + 1, w.w + w.o3(), kWsOut, w.Y, kWsOut, m, 0, 0);
-}
-
-// loss partials into lp, gradient into w.g, of m rows (A0 and Tb filled)
-void ws_backward(desalm_ctx* c, hipStream_t s, int m, double* lp) {
-    WarmStart& w = c->ws;
-    const int nh = w.nh;
-    launch_ws_loss(s, w.Y, w.Tb, m, w.dZ3, lp, kWsLossParts);
-    launch_wgrad(s, w.A2, nh + 1, nh + 1, w.dZ3, kWsOut, kWsOut, m, w.P, w.g + w.o3());
-    launch_dense_bwd(s, w.dZ3, kWsOut, kWsOut, w.w + w.o3(), nh, w.A2, nh + 1, w.dZ2, nh, m);
-    launch_wgrad(s, w.A1, nh + 1, nh + 1, w.dZ2, nh, nh, m, w.P, w.g + w.o2());
-    launch_dense_bwd(s, w.dZ2, nh, nh, w.w + w.o2(), nh, w.A1, nh + 1, w.dZ1, nh, m);
-    launch_wgrad(s, w.A0, kWsIn + 1, kWsIn + 1, w.dZ1, nh, nh, m, w.P, w.g);
+    if (n <= w.lcap) return 0;
+    w.loss = ws_alloc<double>(c, n);
+    if (!w.loss) return -1;
+    w.lcap = n;
+    return 0;
 }
 
 // the warm start of one zone, after the time-level shift
@@ -660,9 +649,9 @@ int ws_start(desalm_ctx* c, hipStream_t s) {
     if (ws_scratch(c, chunk)) return -1;
     for (long r0 = 0; r0 < nint; r0 += chunk) {
         const int m = (int)std::min((long)chunk, nint - r0);
-        launch_ws_features(s, L, c->F, w.q2, w.A0, r0, m, w.stats);
-        ws_forward(c, s, m);
-        launch_ws_apply(s, L, c->F, w.q2, w.Y, r0, m);
+        launch_ws_features(s, L, c->F, w.q2, w.b.A0, r0, m, w.stats);
+        HIPCHK(c, launch_mlp_forward(s, w.b, w.w, w.nh, m));
+        launch_ws_apply(s, L, c->F, w.q2, w.b.Y, r0, m);
     }
     return 0;
 }
@@ -1877,30 +1866,19 @@ int desalm_ws_train(desalm_ctx* c, int iters, int batch, double lr, double* loss
         HIPCHK(c, hipMemcpy(w.stats, st.data(), sizeof(float) * st.size(), hipMemcpyHostToDevice));
         w.have_stats = true;
     }
-    if (w.lcap < (long)iters * kWsLossParts) {
-        w.lpart = ws_alloc<double>(c, (long)iters * kWsLossParts);
-        if (!w.lpart) return -1;
-        w.lcap = (long)iters * kWsLossParts;
-    }
+    if (ws_losses(c, iters)) return -1;
     const float b1 = 0.9f, b2 = 0.999f;
     for (int it = 0; it < iters; it++) {
-        launch_ws_batch(s, w.X, w.T, w.rows, w.A0, w.Tb, batch, w.seed, w.adam_t, w.stats);
-        ws_forward(c, s, batch);
-        ws_backward(c, s, batch, w.lpart + (long)it * kWsLossParts);
+        HIPCHK(c, launch_mlp_train(s, w.b, w.w, w.nh, batch, w.X, w.T, w.rows, w.seed, w.adam_t, w.stats));
         w.adam_t++;
         const float c1 = 1.0f - powf(b1, (float)w.adam_t), c2 = 1.0f - powf(b2, (float)w.adam_t);
-        launch_adam(s, w.w, w.g, w.m, w.v, w.np(), (float)lr, b1, b2, 1e-8f, c1, c2);
+        launch_mlp_grad(s, w.b, w.nh, batch, w.np(), w.g, w.loss + it, w.w, w.m, w.v, (float)lr, b1, b2, 1e-8f, c1, c2);
     }
     HIPCHK(c, hipGetLastError());
     if (loss_out && iters > 0) {
-        std::vector<double> lp((size_t)iters * kWsLossParts);
-        HIPCHK(c, hipMemcpyAsync(lp.data(), w.lpart, sizeof(double) * lp.size(), hipMemcpyDeviceToHost, s));
+        HIPCHK(c, hipMemcpyAsync(loss_out, w.loss, sizeof(double) * iters, hipMemcpyDeviceToHost, s));
         HIPCHK(c, hipStreamSynchronize(s));
-        for (int it = 0; it < iters; it++) {
-            double t = 0.0;
-            for (int b = 0; b < kWsLossParts; b++) t += lp[(size_t)it * kWsLossParts + b];
-            loss_out[it] = t / ((double)batch * kWsComp);
-        }
+        for (int it = 0; it < iters; it++) loss_out[it] = loss_out[it] / ((double)batch * kWsComp);
     }
     HIPCHK(c, hipStreamSynchronize(s));
     return 0;
@@ -2004,10 +1982,9 @@ int desalm_mlp_forward(desalm_ctx* c, const float* x, int64_t m, float* y) {
         for (int f = 0; f < kWsIn; f++) a[(size_t)r * (kWsIn + 1) + f] = x[r * kWsIn + f];
         a[(size_t)r * (kWsIn + 1) + kWsIn] = 1.0f;
     }
-    HIPCHK(c, hipMemcpyAsync(w.A0, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, s));
-    ws_forward(c, s, (int)m);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(y, w.Y, sizeof(float) * m * kWsOut, hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipMemcpyAsync(w.b.A0, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, s));
+    HIPCHK(c, launch_mlp_forward(s, w.b, w.w, w.nh, (int)m));
+    HIPCHK(c, hipMemcpyAsync(y, w.b.Y, sizeof(float) * m * kWsOut, hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
     return 0;
 }
@@ -2020,31 +1997,23 @@ int desalm_mlp_loss_grad(desalm_ctx* c, const float* x, const float* t, int64_t 
     HIPCHK(c, hipSetDevice(c->device));
     hipStream_t s = c->stream;
     if (ws_scratch(c, (int)m)) return -1;
-    if (w.lcap < kWsLossParts) {
-        w.lpart = ws_alloc<double>(c, kWsLossParts);
-        if (!w.lpart) return -1;
-        w.lcap = kWsLossParts;
-    }
-    double* lp = w.lpart;
+    if (ws_losses(c, 1)) return -1;
     std::vector<float> a((size_t)m * (kWsIn + 1));
     for (long r = 0; r < m; r++) {
         for (int f = 0; f < kWsIn; f++) a[(size_t)r * (kWsIn + 1) + f] = x[r * kWsIn + f];
         a[(size_t)r * (kWsIn + 1) + kWsIn] = 1.0f;
     }
-    HIPCHK(c, hipMemcpyAsync(w.A0, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, s));
-    HIPCHK(c, hipMemcpyAsync(w.Tb, t, sizeof(float) * m * kWsTgt, hipMemcpyHostToDevice, s));
-    ws_forward(c, s, (int)m);
-    ws_backward(c, s, (int)m, lp);
+    HIPCHK(c, hipMemcpyAsync(w.b.A0, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, s));
+    HIPCHK(c, hipMemcpyAsync(w.b.Tb, t, sizeof(float) * m * kWsTgt, hipMemcpyHostToDevice, s));
+    HIPCHK(c, launch_mlp_loss(s, w.b, w.w, w.nh, (int)m));
+    launch_mlp_grad(s, w.b, w.nh, (int)m, w.np(), w.g, w.loss, nullptr, nullptr, nullptr, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f,
+                    1.0f);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(grad, w.g, sizeof(float) * w.np(), hipMemcpyDeviceToHost, s));
-    double hl[kWsLossParts];
-    HIPCHK(c, hipMemcpyAsync(hl, lp, sizeof(hl), hipMemcpyDeviceToHost, s));
+    double hl = 0.0;
+    HIPCHK(c, hipMemcpyAsync(&hl, w.loss, sizeof(hl), hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
-    if (loss) {
-        double tsum = 0.0;
-        for (int b = 0; b < kWsLossParts; b++) tsum += hl[b];
-        *loss = tsum / ((double)m * kWsComp);
-    }
+    if (loss) *loss = hl / ((double)m * kWsComp);
     return 0;
 }
 

@@ -173,6 +173,13 @@ constexpr int kWsMaxHidden = 64;
 struct WsQ {
     double* q[5];  // q^(n-2), fine level
 };
+// device matrices of the network's passes, row-major: inputs (ld kWsIn + 1),
+// hidden activations (ld hidden + 1), outputs, scaled targets, the gradients
+// of the three layers' products, weight-gradient partials and loss partials
+struct MlpBuf {
+    float *A0, *A1, *A2, *Y, *Tb, *dZ3, *dZ2, *dZ1, *P;
+    double* lpart;
+};
 
 // Random-flow-generator inflow (k_rfg.hip): N random Fourier modes and, per
 // (j, k) of the inflow plane (index j + nj k), the mean velocity, the
@@ -328,21 +335,19 @@ void launch_gtsv_batch(hipStream_t s, int n, int nsys, double* dl, double* d, do
 
 void launch_ws_sample(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, float* X, float* T, long m,
                       unsigned long long seed, long step);
-void launch_ws_batch(hipStream_t s, const float* X, const float* T, long n, float* Xb, float* Tb, int m,
-                     unsigned long long seed, long it, const float* stats);
 void launch_ws_features(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, float* X, long r0, long m,
                         const float* stats);
 void launch_ws_apply(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* Y, long r0, long m);
-void launch_dense(hipStream_t s, const float* A, int lda, int K1, const float* W, int N, float* Y, int ldy, int M,
-                  int act, int ones);
-void launch_dense_bwd(hipStream_t s, const float* dZ, int ldz, int N, const float* W, int K, const float* Aprev,
-                      int lda, float* dA, int ldd, int M);
+hipError_t launch_mlp_forward(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M);
+hipError_t launch_mlp_loss(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M);
+hipError_t launch_mlp_train(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M, const float* X,
+                            const float* T, long nsrc, unsigned long long seed, long it, const float* stats);
 int wgrad_parts(int M);
-void launch_wgrad(hipStream_t s, const float* A, int lda, int K1, const float* dZ, int ldz, int N, int M, float* P,
-                  float* G);
-void launch_ws_loss(hipStream_t s, const float* Y, const float* T, int M, float* dZ, double* part, int nparts);
-void launch_adam(hipStream_t s, float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2,
-                 float eps, float c1, float c2);
+int mlp_tiles(int M);
+// weight gradients of the tiles' rows into g, the loss sum into *loss, and the
+// Adam update of w (null: none)
+void launch_mlp_grad(hipStream_t s, const MlpBuf& A, int nh, int M, int np, float* g, double* loss, float* w, float* m,
+                     float* v, float lr, float b1, float b2, float eps, float c1, float c2);
 void launch_colstats(hipStream_t s, const float* X, int ld, int nc, long n, double* part, int nparts);
 
 }  // namespace desalm

@@ -15,10 +15,10 @@
 // pseudo-iterations then run to the same tolerance as from any other start,
 // so the warm start only changes how many of them are needed.
 //
-// Everything is FP32 and written here: the feature gather, the dense layers
-// (64 x 64 output tiles, the whole reduction dimension staged in LDS), the
-// backward pass (data gradients with the same tiling, weight gradients as
-// per-chunk partial products summed in a fixed order), the loss and Adam.
+// Everything is FP32 and written here: the feature gather, the layers on tiles
+// of 64 rows that stay in LDS from the input to the output gradient, weight
+// gradients as per-chunk partial products summed in a fixed order, the loss
+// and Adam.
 // Every layer's weights are one (K + 1) x N row-major matrix whose last row
 // is the bias, and every activation matrix carries a trailing column of ones,
 // so a layer is a single product.
@@ -28,8 +28,7 @@ namespace desalm {
 
 namespace {
 
-constexpr int kBM = 64;     // rows (samples) per output tile
-constexpr int kBN = 64;     // columns per output tile
+constexpr int kBM = 64;     // rows (samples) per tile
 constexpr int kKMax = 96;   // largest K + 1 a layer may have
 constexpr int kWgRows = 512;  // rows per weight-gradient partial
 
@@ -112,21 +111,6 @@ __global__ void k_ws_sample(Level L, Fields F, WsQ Q, float* X, float* T, long m
     ws_row(L, F, Q.q, t, X + r * (kWsIn + 1), T + r * kWsTgt, nullptr, nullptr);
 }
 
-// training batch: rows drawn from the first n rows of the sample buffer;
-// features standardised, targets divided by the per-component scale
-__global__ void k_ws_batch(const float* X, const float* T, long n, float* Xb, float* Tb, int m,
-                           unsigned long long seed, long it, const float* stats) {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (r >= m) return;
-    const long src = (long)(mix3(seed ^ 0x5851F42D4C957F2Dull, (unsigned long long)it, (unsigned long long)r) % n);
-    const float* mu = stats;
-    const float* isd = stats + kWsIn;
-    const float* sc = stats + 2 * kWsIn;
-    for (int f = 0; f < kWsIn; f++) Xb[(long)r * (kWsIn + 1) + f] = (X[src * (kWsIn + 1) + f] - mu[f]) * isd[f];
-    Xb[(long)r * (kWsIn + 1) + kWsIn] = 1.0f;
-    for (int e = 0; e < kWsTgt; e++) Tb[(long)r * kWsTgt + e] = T[src * kWsTgt + e] / sc[e % kWsComp];
-}
-
 // inference features of interior ordinals r0 .. r0 + m - 1, standardised
 // when stats is not null
 __global__ void k_ws_features(Level L, Fields F, WsQ Q, float* X, long r0, long m, const float* stats) {
@@ -157,187 +141,379 @@ __global__ void k_ws_apply(Level L, Fields F, WsQ Q, const float* Y, long r0, lo
     }
 }
 
-// Y[:, 0:N] = act(A[:, 0:K1] W), W (K1 x N) row-major; act 1 = tanh.
-// With ones, Y[:, N] = 1.  256 threads, one 64 x 64 tile, 4 x 4 per thread.
-__global__ void __launch_bounds__(256) k_dense(const float* A, int lda, int K1, const float* W, int N, float* Y,
-                                               int ldy, int M, int act, int ones) {
-    __shared__ float As[kKMax][kBM];
-    __shared__ float Ws[kKMax][kBN];
-    const int tid = (int)threadIdx.x;
-    const int r0 = (int)blockIdx.x * kBM, c0 = (int)blockIdx.y * kBN;
-    for (int e = tid; e < kBM * K1; e += 256) {
-        const int row = e / K1, col = e % K1;
-        As[col][row] = (r0 + row < M) ? A[(long)(r0 + row) * lda + col] : 0.0f;
+// ---- the network on tiles of 64 rows ----
+// A workgroup keeps a tile's activations and the weights of all three layers
+// in LDS, so a training step is three launches: k_mlp_tile (batch gather,
+// forward pass, loss, data gradients), k_wgrad (weight gradients of all
+// layers) and k_grad_sum (their partials summed, Adam).  As one launch per
+// layer and direction (fourteen) a step of 16384 rows, 32 hidden units, took
+// 400 us: 92 us for each of three weight gradients, whose 32 workgroups
+// (one per 512 rows) left seven eighths of the CUs idle, and 4.5 us or more
+// for each launch; in three launches it takes 51 us (29, 18 and 5), most of it
+// latency: one tile per CU walks its layers in sequence.  Every sum keeps its
+// order (products over k ascending; rows ascending inside a part of 512,
+// parts ascending), so results are the same bits.
+constexpr int kLd = kBM + 4;  // row stride of the transposed activations [k][row]: float4 reads, few bank conflicts
+
+// floats of LDS: activations of the input and of both hidden layers, and the
+// weights of the three layers with rows padded to an odd count (the backward
+// pass reads them along k).  The gradients of the outputs and of the second
+// hidden layer reuse the input's space.
+struct MlpLds {
+    int ld, w1, w2, w3, a1, a2, total;
+    __host__ __device__ explicit MlpLds(int nh) {
+        ld = nh | 1;
+        w1 = kKMax * kLd;
+        w2 = w1 + (kWsIn + 1) * ld;
+        w3 = w2 + (nh + 1) * ld;
+        a1 = (w3 + (nh + 1) * (kWsOut | 1) + 3) & ~3;
+        a2 = a1 + (nh + 1) * kLd;
+        total = a2 + (nh + 1) * kLd;
     }
-    for (int e = tid; e < K1 * kBN; e += 256) {
-        const int k = e / kBN, n = e % kBN;
-        Ws[k][n] = (c0 + n < N) ? W[(long)k * N + c0 + n] : 0.0f;
-    }
-    __syncthreads();
-    const int tr = tid / 16, tc = tid % 16;
-    float acc[4][4] = {};
+};
+static_assert((kWsOut + kWsMaxHidden) * kLd <= kKMax * kLd, "gradients fit the input's space");
+
+// acc[u][v] = sum over k < K1 of A[k][4 tr + u] W[k][CT tc + v], k ascending
+template <int CT>
+__device__ __forceinline__ void tile_product(const float* A, int K1, const float* W, int ld, int N, int tr, int tc,
+                                             float (&acc)[4][CT]) {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int v = 0; v < CT; v++) acc[u][v] = 0.0f;
+    int col[CT];
+#pragma unroll
+    for (int v = 0; v < CT; v++) col[v] = min(tc * CT + v, N - 1);
+#pragma unroll 8
     for (int k = 0; k < K1; k++) {
-        float a[4], w[4];
+        const float4 a = *reinterpret_cast<const float4*>(A + k * kLd + 4 * tr);
+        float w[CT];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            a[u] = As[k][tr * 4 + u];
-            w[u] = Ws[k][tc * 4 + u];
+        for (int v = 0; v < CT; v++) w[v] = W[k * ld + col[v]];
+#pragma unroll
+        for (int v = 0; v < CT; v++) {
+            acc[0][v] = fmaf(a.x, w[v], acc[0][v]);
+            acc[1][v] = fmaf(a.y, w[v], acc[1][v]);
+            acc[2][v] = fmaf(a.z, w[v], acc[2][v]);
+            acc[3][v] = fmaf(a.w, w[v], acc[3][v]);
         }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[u][v] = fmaf(a[u], w[v], acc[u][v]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int row = r0 + tr * 4 + u;
-        if (row >= M) continue;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int col = c0 + tc * 4 + v;
-            if (col < N) Y[(long)row * ldy + col] = act ? tanhf(acc[u][v]) : acc[u][v];
-        }
-        if (ones && blockIdx.y == 0 && tc == 0) Y[(long)row * ldy + N] = 1.0f;
     }
 }
 
-// dA[:, 0:K] = (dZ W[0:K, :]^T) * (1 - Aprev^2): the gradient through a
-// layer (without its bias row) and the tanh that produced Aprev
-__global__ void __launch_bounds__(256) k_dense_bwd(const float* dZ, int ldz, int N, const float* W, int K,
-                                                   const float* Aprev, int lda, float* dA, int ldd, int M) {
-    __shared__ float Zs[kBN][kBM];
-    __shared__ float Wt[kBN][kBN];
-    const int tid = (int)threadIdx.x;
-    const int r0 = (int)blockIdx.x * kBM, c0 = (int)blockIdx.y * kBN;
-    for (int e = tid; e < kBM * N; e += 256) {
-        const int row = e / N, col = e % N;
-        Zs[col][row] = (r0 + row < M) ? dZ[(long)(r0 + row) * ldz + col] : 0.0f;
-    }
-    for (int e = tid; e < N * kBN; e += 256) {
-        const int n = e / kBN, k = e % kBN;
-        Wt[n][k] = (c0 + k < K) ? W[(long)(c0 + k) * N + n] : 0.0f;
-    }
-    __syncthreads();
+// B[n][row] = tanh(A W), n < N, and the ones column B[N]
+template <int CT>
+__device__ __forceinline__ void tile_layer(const float* A, int K1, const float* W, int ld, int N, float* B, int tid) {
     const int tr = tid / 16, tc = tid % 16;
-    float acc[4][4] = {};
+    float acc[4][CT];
+    tile_product<CT>(A, K1, W, ld, N, tr, tc, acc);
+#pragma unroll
+    for (int v = 0; v < CT; v++) {
+        const int n = tc * CT + v;
+        if (n < N)
+            *reinterpret_cast<float4*>(B + n * kLd + 4 * tr) =
+                make_float4(tanhf(acc[0][v]), tanhf(acc[1][v]), tanhf(acc[2][v]), tanhf(acc[3][v]));
+    }
+    if (tc == 0) *reinterpret_cast<float4*>(B + N * kLd + 4 * tr) = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+}
+
+// G[k][row] = (sum over n of Z[n][row] W[k][n], n ascending) (1 - A[k][row]^2)
+// for k < K: the gradient through a layer (without its bias row) and the tanh
+// that produced A; also stored row-major in Gg (ld K).  G null: Gg only.
+template <int CT>
+__device__ __forceinline__ void tile_back(const float* Z, int N, const float* W, int ld, int K, const float* A,
+                                          float* G, float* Gg, int r0, int M, int tid) {
+    const int tr = tid / 16, tc = tid % 16;
+    int row[CT];
+#pragma unroll
+    for (int v = 0; v < CT; v++) row[v] = min(tc * CT + v, K - 1) * ld;
+    float acc[4][CT] = {};
+#pragma unroll 8
     for (int n = 0; n < N; n++) {
-        float a[4], w[4];
+        const float4 z = *reinterpret_cast<const float4*>(Z + n * kLd + 4 * tr);
+#pragma unroll
+        for (int v = 0; v < CT; v++) {
+            const float w = W[row[v] + n];
+            acc[0][v] = fmaf(z.x, w, acc[0][v]);
+            acc[1][v] = fmaf(z.y, w, acc[1][v]);
+            acc[2][v] = fmaf(z.z, w, acc[2][v]);
+            acc[3][v] = fmaf(z.w, w, acc[3][v]);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < CT; v++) {
+        const int k = tc * CT + v;
+        if (k >= K) continue;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            a[u] = Zs[n][tr * 4 + u];
-            w[u] = Wt[n][tc * 4 + u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[u][v] = fmaf(a[u], w[v], acc[u][v]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int row = r0 + tr * 4 + u;
-        if (row >= M) continue;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int col = c0 + tc * 4 + v;
-            if (col < K) {
-                const float ap = Aprev[(long)row * lda + col];
-                dA[(long)row * ldd + col] = acc[u][v] * (1.0f - ap * ap);
-            }
+            const float ap = A[k * kLd + 4 * tr + u];
+            const float g = acc[u][v] * (1.0f - ap * ap);
+            if (G) G[k * kLd + 4 * tr + u] = g;
+            if (r0 + 4 * tr + u < M) Gg[(long)(r0 + 4 * tr + u) * K + k] = g;
         }
     }
 }
 
-// partial weight gradient of rows [g kWgRows, (g + 1) kWgRows):
-// P[g][k][n] = sum_r A[r][k] dZ[r][n], k < K1 (the ones column gives the bias row)
-__global__ void __launch_bounds__(256) k_wgrad_part(const float* A, int lda, int K1, const float* dZ, int ldz,
-                                                    int N, int M, float* P) {
-    __shared__ float As[kBM][kKMax];
-    __shared__ float Zs[kBM][kBN];
+// 64 rows [64 blockIdx, ...) of M through the network.
+//   kTileForward: rows A.A0 -> outputs A.Y
+//   kTileLoss:    rows A.A0, scaled targets A.Tb -> activations and gradients of every layer (for k_wgrad),
+//                 loss partial of the tile
+//   kTileTrain:   the same on rows drawn from the first nsrc rows of the sample buffer (X, T; standardised
+//                 here, the drawn rows stored in A.A0)
+// Loss: e_c = y_a,c d1_c + y_b,c d2_c - r_c in units of the per-component
+// scale, mean over rows and components of e^2; dZ3 = d loss / d y.
+enum { kTileForward, kTileLoss, kTileTrain };
+template <int MODE, int CT>
+__global__ void __launch_bounds__(256) k_mlp_tile(MlpBuf A, const float* w, int nh, int M, const float* X,
+                                                  const float* T, long nsrc, unsigned long long seed, long it,
+                                                  const float* stats) {
+    extern __shared__ __align__(16) float smem_mlp[];
+    __shared__ long s_src[kBM];
+    __shared__ double s_red[256];
+    const MlpLds O(nh);
+    float* s0 = smem_mlp;
     const int tid = (int)threadIdx.x;
-    const int rbeg = (int)blockIdx.x * kWgRows;
-    const int rend = min(M, rbeg + kWgRows);
-    const int nout = K1 * N;
-    constexpr int kPer = (kKMax * kBN + 255) / 256;
-    float acc[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; j++) acc[j] = 0.0f;
-    for (int rt = rbeg; rt < rend; rt += kBM) {
-        const int nr = min(kBM, rend - rt);
+    const int r0 = (int)blockIdx.x * kBM;
+    constexpr int K1 = kWsIn + 1;
+    if (MODE == kTileTrain) {
+        if (tid < kBM)
+            s_src[tid] = (long)(mix3(seed ^ 0x5851F42D4C957F2Dull, (unsigned long long)it,
+                                     (unsigned long long)(r0 + tid)) % (unsigned long long)nsrc);
         __syncthreads();
-        for (int e = tid; e < kBM * K1; e += 256) {
-            const int row = e / K1, col = e % K1;
-            As[row][col] = row < nr ? A[(long)(rt + row) * lda + col] : 0.0f;
-        }
-        for (int e = tid; e < kBM * N; e += 256) {
-            const int row = e / N, col = e % N;
-            Zs[row][col] = row < nr ? dZ[(long)(rt + row) * ldz + col] : 0.0f;
-        }
-        __syncthreads();
+    }
+    constexpr int kLossPer = (kBM * kWsComp + 255) / 256;
+    float tgt[kLossPer][3], tsc[kLossPer];
+    // the rows: 32 threads along a row, 8 rows at a time, every load issued
+    // before the first use
+    {
+        constexpr int NC = K1 / 32, NR = kBM / 8;
+        static_assert(K1 % 32 == 0, "whole groups of 32 columns");
+        const int cx = tid % 32, rx = tid / 32;
+        float v[NR][NC];
 #pragma unroll
-        for (int j = 0; j < kPer; j++) {
-            const int o = tid + 256 * j;
-            if (o < nout) {
-                const int k = o / N, n = o % N;
-                float s = acc[j];
-                for (int r = 0; r < nr; r++) s = fmaf(As[r][k], Zs[r][n], s);
-                acc[j] = s;
+        for (int r = 0; r < NR; r++) {
+            const int row = rx + 8 * r;
+            const bool in = r0 + row < M;
+            const float* src = MODE == kTileTrain ? X + s_src[row] * K1 : A.A0 + (long)(in ? r0 + row : 0) * K1;
+#pragma unroll
+            for (int c = 0; c < NC; c++) v[r][c] = src[cx + 32 * c];
+        }
+        // the targets of this thread's (row, component) pairs as well
+        if (MODE != kTileForward) {
+#pragma unroll
+            for (int q = 0; q < kLossPer; q++) {
+                const int e = tid + 256 * q, row = e % kBM, c = min(e / kBM, kWsComp - 1);
+                const float* t = MODE == kTileTrain ? T + s_src[row] * kWsTgt
+                                                    : A.Tb + (long)min(r0 + row, M - 1) * kWsTgt;
+#pragma unroll
+                for (int u = 0; u < 3; u++) tgt[q][u] = t[u * kWsComp + c];
+                if (MODE == kTileTrain) tsc[q] = stats[2 * kWsIn + c];
+            }
+        }
+        float mu[NC], isd[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int col = min(cx + 32 * c, kWsIn - 1);
+            mu[c] = MODE == kTileTrain ? stats[col] : 0.0f;
+            isd[c] = MODE == kTileTrain ? stats[kWsIn + col] : 0.0f;
+        }
+        for (int k = rx; k < K1; k += 8)
+            for (int n = cx; n < nh; n += 32) smem_mlp[O.w1 + k * O.ld + n] = w[k * nh + n];
+        const float* w2 = w + K1 * nh;
+        const float* w3 = w2 + (nh + 1) * nh;
+        for (int k = rx; k <= nh; k += 8) {
+            for (int n = cx; n < nh; n += 32) smem_mlp[O.w2 + k * O.ld + n] = w2[k * nh + n];
+            if (cx < kWsOut) smem_mlp[O.w3 + k * (kWsOut | 1) + cx] = w3[k * kWsOut + cx];
+        }
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int row = rx + 8 * r;
+            const bool in = r0 + row < M;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const int col = cx + 32 * c;
+                float x = v[r][c];
+                if (MODE == kTileTrain) {
+                    x = col < kWsIn ? (x - mu[c]) * isd[c] : 1.0f;
+                    if (in) A.A0[(long)(r0 + row) * K1 + col] = x;
+                }
+                s0[col * kLd + row] = in ? x : 0.0f;
             }
         }
     }
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-        const int o = tid + 256 * j;
-        if (o < nout) P[(long)blockIdx.x * nout + o] = acc[j];
-    }
-}
-
-// G[o] = sum over the np partials, in order
-__global__ void k_sum_parts(const float* P, int np, int nout, float* G) {
-    const int o = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (o >= nout) return;
-    float s = 0.0f;
-    for (int g = 0; g < np; g++) s += P[(long)g * nout + o];
-    G[o] = s;
-}
-
-// Loss of the coefficient form, in units of the per-component scale:
-// e_c = y_a,c d1_c + y_b,c d2_c - r_c, loss = mean over rows and components
-// of e^2; dZ = d loss / d y; per-block partial sums of e^2.
-__global__ void __launch_bounds__(256) k_ws_loss(const float* Y, const float* T, int M, float* dZ, double* part) {
-    __shared__ double sh[256];
-    const long tot = (long)M * kWsComp;
-    double s = 0.0;
-    const float scale = 2.0f / (float)tot;
-    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < tot; e += (long)gridDim.x * 256) {
-        const long r = e / kWsComp;
-        const int c = (int)(e % kWsComp);
-        const float* t = T + r * kWsTgt;
-        const float* y = Y + r * kWsOut;
-        const float d1 = t[kWsComp + c], d2 = t[2 * kWsComp + c];
-        const float err = fmaf(y[c], d1, y[kWsComp + c] * d2) - t[c];
-        dZ[r * kWsOut + c] = scale * err * d1;
-        dZ[r * kWsOut + kWsComp + c] = scale * err * d2;
-        s += (double)err * (double)err;
-    }
-    sh[threadIdx.x] = s;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    tile_layer<CT>(s0, K1, smem_mlp + O.w1, O.ld, nh, smem_mlp + O.a1, tid);
+    __syncthreads();
+    tile_layer<CT>(smem_mlp + O.a1, nh + 1, smem_mlp + O.w2, O.ld, nh, smem_mlp + O.a2, tid);
+    __syncthreads();
+    // the output layer: y into the input's space (dead by now), [c][row]
+    {
+        const int tr = tid / 16, tc = tid % 16;
+        float acc[4][1];
+        tile_product<1>(smem_mlp + O.a2, nh + 1, smem_mlp + O.w3, kWsOut | 1, kWsOut, tr, tc, acc);
+        if (tc < kWsOut) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if (MODE == kTileForward) {
+                    if (r0 + 4 * tr + u < M) A.Y[(long)(r0 + 4 * tr + u) * kWsOut + tc] = acc[u][0];
+                } else {
+                    s0[tc * kLd + 4 * tr + u] = acc[u][0];
+                }
+            }
+        }
+    }
+    if (MODE == kTileForward) return;
+    // activations of the hidden layers for k_wgrad
+    for (int row = tid / 32; row < kBM && r0 + row < M; row += 8)
+        for (int col = tid % 32; col <= nh; col += 32) {
+            A.A1[(long)(r0 + row) * (nh + 1) + col] = smem_mlp[O.a1 + col * kLd + row];
+            A.A2[(long)(r0 + row) * (nh + 1) + col] = smem_mlp[O.a2 + col * kLd + row];
+        }
+    __syncthreads();
+    double s = 0.0;
+    const float scale = 2.0f / (float)((long)M * kWsComp);
+#pragma unroll
+    for (int q = 0; q < kLossPer; q++) {
+        const int e = tid + 256 * q, row = e % kBM, c = e / kBM;
+        if (c >= kWsComp) continue;
+        float za = 0.0f, zb = 0.0f;
+        if (r0 + row < M) {
+            const float r = MODE == kTileTrain ? tgt[q][0] / tsc[q] : tgt[q][0];
+            const float d1 = MODE == kTileTrain ? tgt[q][1] / tsc[q] : tgt[q][1];
+            const float d2 = MODE == kTileTrain ? tgt[q][2] / tsc[q] : tgt[q][2];
+            const float err = fmaf(s0[c * kLd + row], d1, s0[(kWsComp + c) * kLd + row] * d2) - r;
+            za = scale * err * d1;
+            zb = scale * err * d2;
+            s += (double)err * (double)err;
+            A.dZ3[(long)(r0 + row) * kWsOut + c] = za;
+            A.dZ3[(long)(r0 + row) * kWsOut + kWsComp + c] = zb;
+        }
+        // only this thread reads or writes these two entries before the barrier
+        s0[c * kLd + row] = za;
+        s0[(kWsComp + c) * kLd + row] = zb;
+    }
+    s_red[tid] = s;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if (tid < h) s_red[tid] += s_red[tid + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    if (tid == 0) A.lpart[blockIdx.x] = s_red[0];
+    tile_back<CT>(s0, kWsOut, smem_mlp + O.w3, kWsOut | 1, nh, smem_mlp + O.a2, s0 + kWsOut * kLd, A.dZ2, r0, M, tid);
+    __syncthreads();
+    tile_back<CT>(s0 + kWsOut * kLd, nh, smem_mlp + O.w2, O.ld, nh, smem_mlp + O.a1, nullptr, A.dZ1, r0, M, tid);
 }
 
-__global__ void k_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-    const int o = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (o >= n) return;
-    const float gi = g[o];
-    const float mi = b1 * m[o] + (1.0f - b1) * gi;
-    const float vi = b2 * v[o] + (1.0f - b2) * gi * gi;
-    m[o] = mi;
-    v[o] = vi;
-    w[o] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// Partial weight gradients of rows [kWgRows blockIdx.x, ...) of all three
+// layers: P[part][offset of the layer + k N + n] = sum_r act[r][k] dZ[r][n]
+// (the ones column gives the bias row).  blockIdx.y walks the layers' tiles of
+// kWgK x kWgN outputs, so a batch of 16384 rows is 384 workgroups.
+constexpr int kWgK = 16, kWgN = 32, kWgTile = 128;
+__host__ __device__ inline int wg_tiles(int K1, int N) { return ((K1 + kWgK - 1) / kWgK) * ((N + kWgN - 1) / kWgN); }
+__global__ void __launch_bounds__(128) k_wgrad(MlpBuf A, int nh, int M, int np) {
+    __shared__ float As[kWgTile][kWgK];
+    __shared__ float Zs[kWgTile][kWgN];
+    int tile = (int)blockIdx.y;
+    const int n1 = wg_tiles(kWsIn + 1, nh), n2 = wg_tiles(nh + 1, nh);
+    const float *act, *dz;
+    int K1, N, base;
+    if (tile < n1) {
+        act = A.A0; dz = A.dZ1; K1 = kWsIn + 1; N = nh; base = 0;
+    } else if (tile < n1 + n2) {
+        tile -= n1;
+        act = A.A1; dz = A.dZ2; K1 = nh + 1; N = nh; base = (kWsIn + 1) * nh;
+    } else {
+        tile -= n1 + n2;
+        act = A.A2; dz = A.dZ3; K1 = nh + 1; N = kWsOut; base = (kWsIn + 1 + nh + 1) * nh;
+    }
+    const int tk = (K1 + kWgK - 1) / kWgK;
+    const int k0 = (tile % tk) * kWgK, n0 = (tile / tk) * kWgN;
+    const int tid = (int)threadIdx.x;
+    const int kx = 2 * (tid / 16), nx = 2 * (tid % 16);
+    const int rbeg = (int)blockIdx.x * kWgRows, rend = min(M, rbeg + kWgRows);
+    // the next tile's rows are loaded while the current one is summed, at
+    // clamped addresses (no branch around a load)
+    constexpr int QA = kWgTile * kWgK / 128, QZ = kWgTile * kWgN / 128;
+    float av[QA], zv[QZ];
+    const int ka = k0 + tid % kWgK, nz = n0 + tid % kWgN;  // columns of this thread's loads
+    const float* ap = act + min(ka, K1 - 1);
+    const float* zp = dz + min(nz, N - 1);
+    const int ra = tid / kWgK, rz = tid / kWgN;
+    auto load = [&](int rt) {
+#pragma unroll
+        for (int q = 0; q < QA; q++) av[q] = ap[(long)min(rt + ra + 128 / kWgK * q, rend - 1) * K1];
+#pragma unroll
+        for (int q = 0; q < QZ; q++) zv[q] = zp[(long)min(rt + rz + 128 / kWgN * q, rend - 1) * N];
+    };
+    float acc[2][2] = {};
+    load(rbeg);
+    for (int rt = rbeg; rt < rend; rt += kWgTile) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < QA; q++) (&As[0][0])[tid + 128 * q] = rt + ra + 128 / kWgK * q < rend ? av[q] : 0.0f;
+#pragma unroll
+        for (int q = 0; q < QZ; q++) (&Zs[0][0])[tid + 128 * q] = rt + rz + 128 / kWgN * q < rend ? zv[q] : 0.0f;
+        load(rt + kWgTile);
+        __syncthreads();
+        // rows past the part's end are zero on both sides
+#pragma unroll 16
+        for (int r = 0; r < kWgTile; r++) {
+            const float2 a = *reinterpret_cast<const float2*>(&As[r][kx]);
+            const float2 z = *reinterpret_cast<const float2*>(&Zs[r][nx]);
+            acc[0][0] = fmaf(a.x, z.x, acc[0][0]);
+            acc[0][1] = fmaf(a.x, z.y, acc[0][1]);
+            acc[1][0] = fmaf(a.y, z.x, acc[1][0]);
+            acc[1][1] = fmaf(a.y, z.y, acc[1][1]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++)
+            if (k0 + kx + u < K1 && n0 + nx + v < N)
+                A.P[(long)blockIdx.x * np + base + (k0 + kx + u) * N + n0 + nx + v] = acc[u][v];
+}
+
+struct AdamArgs {
+    float *w, *m, *v;  // null w: no update
+    float lr, b1, b2, eps, c1, c2;
+};
+
+// g[o] = sum over the parts, ascending, then the Adam update of parameter o;
+// the last workgroup sums the loss partials of the row tiles into loss
+__global__ void __launch_bounds__(256) k_grad_sum(const float* P, int nparts, int np, float* g, AdamArgs a,
+                                                  const double* lpart, int ntiles, double* loss) {
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double s_red[256];
+        double s = 0.0;
+        for (int b = (int)threadIdx.x; b < ntiles; b += 256) s += lpart[b];
+        s_red[threadIdx.x] = s;
+        __syncthreads();
+        for (int h = 128; h > 0; h >>= 1) {
+            if ((int)threadIdx.x < h) s_red[threadIdx.x] += s_red[threadIdx.x + h];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *loss = s_red[0];
+        return;
+    }
+    const int o = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (o >= np) return;
+    float s = 0.0f;
+    int p = 0;
+    for (; p + 8 <= nparts; p += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = P[(long)(p + u) * np + o];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; p < nparts; p++) s += P[(long)p * np + o];
+    g[o] = s;
+    if (!a.w) return;
+    const float mi = a.b1 * a.m[o] + (1.0f - a.b1) * s;
+    const float vi = a.b2 * a.v[o] + (1.0f - a.b2) * s * s;
+    a.m[o] = mi;
+    a.v[o] = vi;
+    a.w[o] -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
 }
 
 // per-column sum and sum of squares over n rows (ld columns, first nc used),
@@ -379,11 +555,6 @@ void launch_ws_sample(hipStream_t s, const Level& L, const Fields& F, const WsQ&
     hipLaunchKernelGGL(k_ws_sample, dim3(nblk(m, 128)), dim3(128), 0, s, L, F, Q, X, T, m, seed, step);
 }
 
-void launch_ws_batch(hipStream_t s, const float* X, const float* T, long n, float* Xb, float* Tb, int m,
-                     unsigned long long seed, long it, const float* stats) {
-    hipLaunchKernelGGL(k_ws_batch, dim3(nblk(m, 128)), dim3(128), 0, s, X, T, n, Xb, Tb, m, seed, it, stats);
-}
-
 void launch_ws_features(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, float* X, long r0, long m,
                         const float* stats) {
     hipLaunchKernelGGL(k_ws_features, dim3(nblk(m, 128)), dim3(128), 0, s, L, F, Q, X, r0, m, stats);
@@ -393,34 +564,49 @@ void launch_ws_apply(hipStream_t s, const Level& L, const Fields& F, const WsQ& 
     hipLaunchKernelGGL(k_ws_apply, dim3(nblk(m, 256)), dim3(256), 0, s, L, F, Q, Y, r0, m);
 }
 
-void launch_dense(hipStream_t s, const float* A, int lda, int K1, const float* W, int N, float* Y, int ldy, int M,
-                  int act, int ones) {
-    hipLaunchKernelGGL(k_dense, dim3(nblk(M, kBM), nblk(N, kBN)), dim3(256), 0, s, A, lda, K1, W, N, Y, ldy, M, act,
-                       ones);
+// the tile kernel in one of its modes; the hidden width picks the columns per
+// thread (16 column groups)
+template <int MODE>
+static hipError_t mlp_tile(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M, const float* X,
+                           const float* T, long nsrc, unsigned long long seed, long it, const float* stats) {
+    const int lds = (int)sizeof(float) * MlpLds(nh).total;
+    const dim3 grid(nblk(M, kBM)), block(256);
+    auto go = [&](auto kernel) {
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, A, w, nh, M, X, T, nsrc, seed, it, stats);
+        return hipGetLastError();
+    };
+    return nh <= 32 ? go(k_mlp_tile<MODE, 2>) : go(k_mlp_tile<MODE, 4>);
 }
 
-void launch_dense_bwd(hipStream_t s, const float* dZ, int ldz, int N, const float* W, int K, const float* Aprev,
-                      int lda, float* dA, int ldd, int M) {
-    hipLaunchKernelGGL(k_dense_bwd, dim3(nblk(M, kBM), nblk(K, kBN)), dim3(256), 0, s, dZ, ldz, N, W, K, Aprev, lda,
-                       dA, ldd, M);
+hipError_t launch_mlp_forward(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M) {
+    return mlp_tile<kTileForward>(s, A, w, nh, M, nullptr, nullptr, 1, 0, 0, nullptr);
+}
+
+hipError_t launch_mlp_loss(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M) {
+    return mlp_tile<kTileLoss>(s, A, w, nh, M, nullptr, nullptr, 1, 0, 0, nullptr);
+}
+
+hipError_t launch_mlp_train(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M, const float* X,
+                            const float* T, long nsrc, unsigned long long seed, long it, const float* stats) {
+    return mlp_tile<kTileTrain>(s, A, w, nh, M, X, T, nsrc, seed, it, stats);
 }
 
 int wgrad_parts(int M) { return (int)nblk(M, kWgRows); }
+int mlp_tiles(int M) { return (int)nblk(M, kBM); }
 
-void launch_wgrad(hipStream_t s, const float* A, int lda, int K1, const float* dZ, int ldz, int N, int M, float* P,
-                  float* G) {
-    const int np = wgrad_parts(M);
-    hipLaunchKernelGGL(k_wgrad_part, dim3(np), dim3(256), 0, s, A, lda, K1, dZ, ldz, N, M, P);
-    hipLaunchKernelGGL(k_sum_parts, dim3(nblk((long)K1 * N, 256)), dim3(256), 0, s, P, np, K1 * N, G);
-}
-
-void launch_ws_loss(hipStream_t s, const float* Y, const float* T, int M, float* dZ, double* part, int nparts) {
-    hipLaunchKernelGGL(k_ws_loss, dim3(nparts), dim3(256), 0, s, Y, T, M, dZ, part);
-}
-
-void launch_adam(hipStream_t s, float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2,
-                 float eps, float c1, float c2) {
-    hipLaunchKernelGGL(k_adam, dim3(nblk(n, 256)), dim3(256), 0, s, w, g, m, v, n, lr, b1, b2, eps, c1, c2);
+void launch_mlp_grad(hipStream_t s, const MlpBuf& A, int nh, int M, int np, float* g, double* loss, float* w, float* m,
+                     float* v, float lr, float b1, float b2, float eps, float c1, float c2) {
+    const int parts = wgrad_parts(M);
+    const int tiles = wg_tiles(kWsIn + 1, nh) + wg_tiles(nh + 1, nh) + wg_tiles(nh + 1, kWsOut);
+    hipLaunchKernelGGL(k_wgrad, dim3(parts, tiles), dim3(128), 0, s, A, nh, M, np);
+    const AdamArgs a{w, m, v, lr, b1, b2, eps, c1, c2};
+    hipLaunchKernelGGL(k_grad_sum, dim3(nblk(np, 256) + 1), dim3(256), 0, s, A.P, parts, np, g, a, A.lpart,
+                       mlp_tiles(M), loss);
 }
 
 void launch_colstats(hipStream_t s, const float* X, int ld, int nc, long n, double* part, int nparts) {

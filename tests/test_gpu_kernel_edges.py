@@ -1,0 +1,35 @@
+"""Kernels at the sizes where their tiling can go wrong (tile edges,
+remainders, the smallest and largest of their range), against the CPU oracle."""
+import numpy as np
+import pytest
+
+import mlp_oracle as mo
+from desalm import cases
+from desalm.lib import Solver
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nh,m", [(1, 1), (2, 63), (16, 64), (31, 65), (32, 511), (33, 512), (48, 513), (64, 1025)])
+def test_mlp_tiles(gpu, nh, m):
+    """Forward pass, loss and gradient at the edges of the 64-row tiles, the
+    512-row weight-gradient parts and the hidden widths (32: two columns per
+    thread, 33: four)."""
+    c = cases.wavy(13, 11, 9, ng=2, itm=2, iters=(1, 2))
+    s = Solver(c.params).load_case(c)
+    s.ws_configure(hidden=nh, samples_per_record=64, capacity=256, seed=3)
+    rng = np.random.default_rng(100 * nh + m)
+    w = rng.normal(0.0, 0.2, mo.param_count(nh)).astype(np.float32)
+    s.ws_params(w)
+    x = rng.normal(size=(m, mo.N_IN)).astype(np.float32)
+    t = rng.normal(size=(m, 3 * mo.N_COMP)).astype(np.float32)
+    w8, x8, t8 = w.astype(np.float64), x.astype(np.float64), t.astype(np.float64)
+    y, yo = s.mlp_forward(x), mo.forward(w8, x8, nh)
+    # FP32 sums of at most 97 products: 97 roundings of 6e-8 of the largest sum
+    assert np.abs(y - yo).max() <= 2e-5 * max(1.0, np.abs(yo).max())
+    loss, g = s.mlp_loss_grad(x, t)
+    lo, go = mo.loss_grad(w8, x8, t8, nh)
+    assert abs(loss - lo) <= 1e-5 * abs(lo)
+    # sums over up to 1025 rows, in order: 1025 roundings of 6e-8
+    assert np.abs(g - go).max() <= 1e-4 * np.abs(go).max()
+    s.close()
