@@ -641,18 +641,11 @@ int ws_start(desalm_ctx* c, hipStream_t s) {
     const Level& L = c->lv[1];
     const long nint = (long)(L.ni - 2) * (L.nj - 2) * (L.nk - 2);
     if (w.mode == DESALM_WS_EXTRAP) {
-        launch_ws_apply(s, L, c->F, w.q2, nullptr, 0, nint);
+        launch_ws_extrap(s, L, c->F, nint);
         return 0;
     }
     if (!w.have_stats) return fail(c, "learned warm start: the network has not been trained (desalm_ws_train)");
-    const int chunk = 1 << 17;
-    if (ws_scratch(c, chunk)) return -1;
-    for (long r0 = 0; r0 < nint; r0 += chunk) {
-        const int m = (int)std::min((long)chunk, nint - r0);
-        launch_ws_features(s, L, c->F, w.q2, w.b.A0, r0, m, w.stats);
-        HIPCHK(c, launch_mlp_forward(s, w.b, w.w, w.nh, m));
-        launch_ws_apply(s, L, c->F, w.q2, w.b.Y, r0, m);
-    }
+    HIPCHK(c, launch_ws_infer(s, L, c->F, w.q2, w.w, w.nh, w.stats, nint));
     return 0;
 }
 

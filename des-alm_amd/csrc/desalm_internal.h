@@ -337,7 +337,10 @@ void launch_ws_sample(hipStream_t s, const Level& L, const Fields& F, const WsQ&
                       unsigned long long seed, long step);
 void launch_ws_features(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, float* X, long r0, long m,
                         const float* stats);
-void launch_ws_apply(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* Y, long r0, long m);
+// the warm start of the m interior nodes: linear extrapolation, or the network
+void launch_ws_extrap(hipStream_t s, const Level& L, const Fields& F, long m);
+hipError_t launch_ws_infer(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* w, int nh,
+                           const float* stats, long m);
 hipError_t launch_mlp_forward(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M);
 hipError_t launch_mlp_loss(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M);
 hipError_t launch_mlp_train(hipStream_t s, const MlpBuf& A, const float* w, int nh, int M, const float* X,

@@ -120,22 +120,14 @@ __global__ void k_ws_features(Level L, Fields F, WsQ Q, float* X, long r0, long 
            stats ? stats + kWsIn : nullptr);
 }
 
-// q(0) = q^n + (1 + y_a) d1 + y_b d2 on interior ordinals r0 .. r0 + m - 1
-// (y = 0 without a network: linear extrapolation); nu~ keeps the floor of the
-// SA update (rhs_sa_bcond.F90:283-287)
-__global__ void k_ws_apply(Level L, Fields F, WsQ Q, const float* Y, long r0, long m) {
+// linear extrapolation 2 q^n - q^(n-1) on the interior; nu~ keeps the floor
+// of the SA update (rhs_sa_bcond.F90:283-287)
+__global__ void k_ws_extrap(Level L, Fields F, long m) {
     const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= m) return;
-    const long g = L.off + interior_node(L, r0 + r);
+    const long g = L.off + interior_node(L, r);
     for (int c = 0; c < kWsComp; c++) {
-        const double qn = F.qn[c][g], qm = F.qnm1[c][g];
-        double v;
-        if (Y) {
-            const double d1 = qn - qm, d2 = qm - Q.q[c][g - L.off];
-            v = qn + (1.0 + (double)Y[r * kWsOut + c]) * d1 + (double)Y[r * kWsOut + kWsComp + c] * d2;
-        } else {
-            v = 2.0 * qn - qm;
-        }
+        double v = 2.0 * F.qn[c][g] - F.qnm1[c][g];
         if (c == 4) v = fmax(1.0e-07, v);
         F.q[c][g] = v;
     }
@@ -516,6 +508,166 @@ __global__ void __launch_bounds__(256) k_grad_sum(const float* P, int nparts, in
     a.w[o] -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
 }
 
+// The learned start of the whole interior in one launch: features of a tile
+// of TM nodes into LDS, the three layers on the tile (4 x 4 outputs per
+// thread, weights resident in LDS), and
+//   q(0) = q^n + (1 + y_a) d1 + y_b d2,  nu~ >= 1e-7,
+// written from there.  A workgroup walks a contiguous run of tiles, so the
+// weights are staged once and the j neighbours of a tile come from its L2.
+// Bound by FP32 and FP64 arithmetic (4458 multiply-adds, 64 tanh and 90 FP64
+// divisions per node with 32 hidden units).  As a feature pass, three layer
+// passes and an apply pass over chunks of 131072 nodes the rows crossed HBM
+// five times and the feature rows were written 96 words apart by adjacent
+// threads: 17 ms for the 9.3 M interior nodes of a 257x193x193 block, 4.1 ms
+// here.  TM = 128 for up to 32 hidden units (8 column groups of 4), 64 above (16): the
+// tile's rows times its column groups fill 256 threads either way.
+// Products run over k ascending and features are rounded as in ws_row.
+template <int TM>
+__device__ __forceinline__ void infer_product(const float* A, int K1, const float* W, int ld, int tr, int tc,
+                                              float (&acc)[4][4]) {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[u][v] = 0.0f;
+#pragma unroll 4
+    for (int k = 0; k < K1; k++) {
+        const float4 a = *reinterpret_cast<const float4*>(A + k * (TM + 4) + 4 * tr);
+        const float4 w = *reinterpret_cast<const float4*>(W + k * ld + 4 * tc);
+        const float av[4] = {a.x, a.y, a.z, a.w}, wv[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[u][v] = fmaf(av[u], wv[v], acc[u][v]);
+    }
+}
+
+template <int TM>
+struct InferLds {
+    static constexpr int NC = TM == 128 ? 32 : 64;  // padded hidden width
+    static constexpr int LA = TM + 4;
+    static constexpr int act = 0;                                // [kKMax][LA]; later both hidden layers and y
+    static constexpr int w1 = kKMax * LA;                        // [96][NC]
+    static constexpr int w2 = w1 + (kWsIn + 1) * NC;             // [NC + 1][NC]
+    static constexpr int w3 = w2 + (NC + 1) * NC;                // [NC + 1][12]
+    static constexpr int total = w3 + (NC + 1) * 12;
+};
+static_assert(2 * 33 + kWsOut <= kKMax, "both hidden layers and y fit the input's rows (32 units)");
+
+template <int TM>
+__global__ void __launch_bounds__(256) k_ws_infer(Level L, Fields F, WsQ Q, const float* w, int nh, const float* stats,
+                                                  long m, int ntiles) {
+    extern __shared__ __align__(16) float smem_mlp[];
+    using O = InferLds<TM>;
+    constexpr int K1 = kWsIn + 1, LA = O::LA, NC = O::NC;
+    __shared__ int s_node[TM];
+    const int tid = (int)threadIdx.x;
+    float* act = smem_mlp + O::act;
+    // weights, columns and rows past the network's zero
+    for (int e = tid; e < K1 * NC; e += 256) {
+        const int k = e / NC, n = e % NC;
+        smem_mlp[O::w1 + e] = n < nh ? w[k * nh + n] : 0.0f;
+    }
+    const float* g2 = w + K1 * nh;
+    const float* g3 = g2 + (nh + 1) * nh;
+    for (int e = tid; e < (nh + 1) * NC; e += 256) {
+        const int k = e / NC, n = e % NC;
+        smem_mlp[O::w2 + e] = n < nh ? g2[k * nh + n] : 0.0f;
+    }
+    for (int e = tid; e < (nh + 1) * 12; e += 256) {
+        const int k = e / 12, n = e % 12;
+        smem_mlp[O::w3 + e] = n < kWsOut ? g3[k * kWsOut + n] : 0.0f;
+    }
+    const int tr = tid / (NC / 4), tc = tid % (NC / 4);
+    // this workgroup's run of tiles
+    const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+    const int t0 = (int)((long)ntiles * lb / gridDim.x), t1 = (int)((long)ntiles * (lb + 1) / gridDim.x);
+    for (int tile = t0; tile < t1; tile++) {
+        const long r0 = (long)tile * TM;
+        __syncthreads();  // the weights, and y of the tile before
+        if (tid < TM) s_node[tid] = (int)interior_node(L, min(r0 + tid, m - 1));
+        __syncthreads();
+        // features: one component of one node per thread and turn (whole
+        // waves share a component)
+        for (int e = tid; e < TM * kWsComp; e += 256) {
+            const int row = e % TM, c = __builtin_amdgcn_readfirstlane(e / TM);
+            const int t = s_node[row], i = t % L.ni;
+            const int st[kWsPts] = {0, -1, 1, -L.ni, L.ni, -L.ni * L.nj, L.ni * L.nj,
+                                    i >= 2 ? -2 : -i, i + 2 <= L.ni - 1 ? 2 : L.ni - 1 - i};
+            const double* a = F.qn[c] + L.off;
+            const double* b = F.qnm1[c] + L.off;
+            const double* d = Q.q[c];
+            double av[kWsPts], bv[kWsPts], dv[kWsPts];
+#pragma unroll
+            for (int s = 0; s < kWsPts; s++) {
+                av[s] = a[t + st[s]];
+                bv[s] = b[t + st[s]];
+                dv[s] = d[t + st[s]];
+            }
+            double v[2 * kWsPts];
+            double ss = 0.0;
+#pragma unroll
+            for (int s = 0; s < kWsPts; s++) {
+                v[2 * s] = av[s] - bv[s];
+                v[2 * s + 1] = bv[s] - dv[s];
+                ss += v[2 * s] * v[2 * s] + v[2 * s + 1] * v[2 * s + 1];
+            }
+            const double rms = sqrt(ss / (2 * kWsPts));
+            const int f0 = c * 2 * kWsPts, fq = kWsComp * 2 * kWsPts + c;
+#pragma unroll
+            for (int q = 0; q < 2 * kWsPts; q++) {
+                const float x = rms > 0.0 ? (float)(v[q] / rms) : 0.0f;
+                act[(f0 + q) * LA + row] = (x - stats[f0 + q]) * stats[kWsIn + f0 + q];
+            }
+            act[fq * LA + row] = ((float)av[0] - stats[fq]) * stats[kWsIn + fq];
+            if (c == 0) act[kWsIn * LA + row] = 1.0f;
+        }
+        __syncthreads();
+        float acc[4][4];
+        infer_product<TM>(act, K1, smem_mlp + O::w1, NC, tr, tc, acc);
+        __syncthreads();  // the input is dead: rows 0 .. nh hold the first hidden layer
+        auto store_layer = [&](float* B) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int n = 4 * tc + v;
+                if (n < nh)
+                    *reinterpret_cast<float4*>(B + n * LA + 4 * tr) =
+                        make_float4(tanhf(acc[0][v]), tanhf(acc[1][v]), tanhf(acc[2][v]), tanhf(acc[3][v]));
+            }
+            if (tc == 0) *reinterpret_cast<float4*>(B + nh * LA + 4 * tr) = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        };
+        store_layer(act);
+        __syncthreads();
+        infer_product<TM>(act, nh + 1, smem_mlp + O::w2, NC, tr, tc, acc);
+        // the second hidden layer beside the first where both fit, else over it
+        constexpr int second = TM == 128 ? 33 : 0;
+        if (second == 0) __syncthreads();
+        float* B2 = act + second * LA;
+        store_layer(B2);
+        __syncthreads();
+        float* y = act + (TM == 128 ? 66 : 65) * LA;  // [10][LA]
+        if (tc < 3) {
+            infer_product<TM>(B2, nh + 1, smem_mlp + O::w3, 12, tr, tc, acc);
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (4 * tc + v < kWsOut)
+                    *reinterpret_cast<float4*>(y + (4 * tc + v) * LA + 4 * tr) =
+                        make_float4(acc[0][v], acc[1][v], acc[2][v], acc[3][v]);
+        }
+        __syncthreads();
+        for (int e = tid; e < TM * kWsComp; e += 256) {
+            const int row = e % TM, c = __builtin_amdgcn_readfirstlane(e / TM);
+            if (r0 + row >= m) continue;
+            const int t = s_node[row];
+            const long g = L.off + t;
+            const double qn = F.qn[c][g], qm = F.qnm1[c][g];
+            const double d1 = qn - qm, d2 = qm - Q.q[c][t];
+            double v = qn + (1.0 + (double)y[c * LA + row]) * d1 + (double)y[(kWsComp + c) * LA + row] * d2;
+            if (c == 4) v = fmax(1.0e-07, v);
+            F.q[c][g] = v;
+        }
+    }
+}
+
 // per-column sum and sum of squares over n rows (ld columns, first nc used),
 // partial per block: part[blockIdx][2 nc]
 __global__ void __launch_bounds__(256) k_colstats(const float* X, int ld, int nc, long n, double* part) {
@@ -560,8 +712,27 @@ void launch_ws_features(hipStream_t s, const Level& L, const Fields& F, const Ws
     hipLaunchKernelGGL(k_ws_features, dim3(nblk(m, 128)), dim3(128), 0, s, L, F, Q, X, r0, m, stats);
 }
 
-void launch_ws_apply(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* Y, long r0, long m) {
-    hipLaunchKernelGGL(k_ws_apply, dim3(nblk(m, 256)), dim3(256), 0, s, L, F, Q, Y, r0, m);
+void launch_ws_extrap(hipStream_t s, const Level& L, const Fields& F, long m) {
+    hipLaunchKernelGGL(k_ws_extrap, dim3(nblk(m, 256)), dim3(256), 0, s, L, F, m);
+}
+
+template <int TM>
+static hipError_t ws_infer(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* w, int nh,
+                           const float* stats, long m) {
+    const int lds = (int)sizeof(float) * InferLds<TM>::total;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_ws_infer<TM>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+    const int ntiles = (int)((m + TM - 1) / TM);
+    // two workgroups per CU (69 KB of LDS each with TM = 128)
+    const unsigned grid = (unsigned)(ntiles < 512 ? ntiles : 512);
+    hipLaunchKernelGGL(k_ws_infer<TM>, dim3(grid), dim3(256), lds, s, L, F, Q, w, nh, stats, m, ntiles);
+    return hipGetLastError();
+}
+
+hipError_t launch_ws_infer(hipStream_t s, const Level& L, const Fields& F, const WsQ& Q, const float* w, int nh,
+                           const float* stats, long m) {
+    return nh <= 32 ? ws_infer<128>(s, L, F, Q, w, nh, stats, m) : ws_infer<64>(s, L, F, Q, w, nh, stats, m);
 }
 
 // the tile kernel in one of its modes; the hidden width picks the columns per

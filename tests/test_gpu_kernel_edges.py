@@ -33,3 +33,34 @@ def test_mlp_tiles(gpu, nh, m):
     # sums over up to 1025 rows, in order: 1025 roundings of 6e-8
     assert np.abs(g - go).max() <= 1e-4 * np.abs(go).max()
     s.close()
+
+
+@pytest.mark.parametrize("nh,dims", [(1, (5, 5, 5)), (32, (34, 6, 6)), (32, (35, 6, 6)), (33, (18, 6, 6)),
+                                     (64, (19, 7, 9))])
+def test_learned_start_tiles(gpu, nh, dims):
+    """The one-launch learned start with interiors of 27, 512 and 528 nodes on
+    128-node tiles (up to 32 hidden units) and 256 and 595 on 64-node tiles."""
+    c = cases.wavy(*dims, ng=1, itm=1, seed=9)
+    s = Solver(c.params).load_case(c)
+    s.ws_configure(hidden=nh, samples_per_record=64, capacity=256, seed=3)
+    q, qn, qnm1, _ = s.get_state()
+    rng = np.random.default_rng(nh)
+    w = rng.normal(0.0, 0.3, mo.param_count(nh)).astype(np.float32)
+    stats = np.concatenate([rng.normal(0.0, 0.3, 95), rng.uniform(0.5, 2.0, 95),
+                            rng.uniform(0.01, 0.1, 5), np.zeros(5)]).astype(np.float32)
+    s.ws_params(w)
+    s.ws_stats(stats)
+    s.ws_mode(Solver.WS_LEARNED)
+    s.set_convergence(0, 0, -8.0, -30.0)
+    s.mg_driver()
+    got = s.get_state()[0]
+    want = mo.warm_start(q, q, qn, qnm1, dims, w.astype(np.float64), nh, stats.astype(np.float64))
+    ext = mo.warm_start(q, q, qn, qnm1, dims)
+    g = mo.interior_index(dims)
+    # the coefficients are FP32 sums of at most 97 products, applied in FP64
+    scale = np.abs(want[g] - ext[g]).max(axis=0)
+    assert (scale > 0).all()
+    assert (np.abs(got[g] - want[g]).max(axis=0) <= 2e-5 * scale + 1e-14).all()
+    rest = np.setdiff1d(np.arange(len(q)), g)
+    assert np.array_equal(got[rest], q[rest])
+    s.close()
