@@ -769,9 +769,11 @@ template <int D, int R, typename S>
 __global__ void __launch_bounds__(512) k_daf_sweep_z(ZoneGrid G, int n, int P, int TI) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    const Level& L = Z.lv[n];
-    const SweepFlags f = sweep_flags(Z.C, D, n);
-    daf_body<D, R, S>(L, Z.F, Z.C, sweep_io<S>(Z.F, D), sweep_lines(L, D, f.ext, P, TI), f.use_b1, f.use_b2,
+    const Level L = Z.lv[n];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    const SweepFlags f = sweep_flags(C, D, n);
+    daf_body<D, R, S>(L, F, C, sweep_io<S>(F, D), sweep_lines(L, D, f.ext, P, TI), f.use_b1, f.use_b2,
                       f.b2_full, f.ext, nullptr, xcd_block(b.bid, b.nblk));
 }
 

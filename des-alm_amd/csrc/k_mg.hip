@@ -542,7 +542,10 @@ __global__ void __launch_bounds__(256) k_nlevel(Level Lc, Level Lf, Fields F, in
 __global__ void __launch_bounds__(256) k_nlevel_z(ZoneGrid G, int n) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    nlevel_body(Z.lv[n], Z.lv[n - 1], Z.F, Z.icrs, Z.jcrs, Z.kcrs, b.bid, b.nblk);
+    const Level Lc = Z.lv[n], Lf = Z.lv[n - 1];
+    const Fields F = Z.F;
+    const int ic = Z.icrs, jc = Z.jcrs, kc = Z.kcrs;
+    nlevel_body(Lc, Lf, F, ic, jc, kc, b.bid, b.nblk);
 }
 __global__ void __launch_bounds__(256) k_prolong_fill(ProlongCtx P, Fields F) {
     prolong_fill_body(P, F, blockIdx.x, gridDim.x);
@@ -551,7 +554,8 @@ __global__ void __launch_bounds__(256) k_prolong_fill_z(ZoneGrid G, int n) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
     const ProlongCtx P{Z.lv[n], Z.lv[n + 1], Z.icrs, Z.jcrs, Z.kcrs};
-    prolong_fill_body(P, Z.F, b.bid, b.nblk);
+    const Fields F = Z.F;
+    prolong_fill_body(P, F, b.bid, b.nblk);
 }
 template <int D, int R>
 __global__ void __launch_bounds__(512) k_rs_sweep(Level L, Fields F, SegShape sh, double epn) {
@@ -561,7 +565,9 @@ template <int D, int R>
 __global__ void __launch_bounds__(512) k_rs_sweep_z(ZoneGrid G, int n, int P, int TI) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    rs_sweep_body<D, R>(Z.lv[n], Z.F, seg_lines(Z.lv[n], D, P, TI), Z.C.ep[1][D], xcd_block(b.bid, b.nblk));
+    const Level L = Z.lv[n];
+    const Fields F = Z.F;
+    rs_sweep_body<D, R>(L, F, seg_lines(L, D, P, TI), Z.C.ep[1][D], xcd_block(b.bid, b.nblk));
 }
 // D = 2 also reads the pinned pressure into F.pfix (bcond_fm.F90:310-322),
 // in the thread of the pinned node's k column (face node tfix) after that
@@ -576,7 +582,10 @@ template <int D>
 __global__ void __launch_bounds__(256) k_bc_fm_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    bc_fm_body<D>(Z.lv[1], Z.F, Z.C, b.bid);
+    const Level L = Z.lv[1];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    bc_fm_body<D>(L, F, C, b.bid);
 }
 // one thread per zone
 __global__ void k_pfix_read_z(const ZoneDesc* __restrict__ z, int nz) {
@@ -586,14 +595,18 @@ __global__ void k_pfix_read_z(const ZoneDesc* __restrict__ z, int nz) {
 __global__ void __launch_bounds__(256) k_pfix_sub(Level L, Fields F) { pfix_sub_body(L, F, blockIdx.x); }
 __global__ void __launch_bounds__(256) k_pfix_sub_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
-    pfix_sub_body(G.z[b.z].lv[1], G.z[b.z].F, b.bid);
+    const Level L = G.z[b.z].lv[1];
+    const Fields F = G.z[b.z].F;
+    pfix_sub_body(L, F, b.bid);
 }
 __global__ void __launch_bounds__(256) k_resid_part(Level L, Fields F, int save, int pfix) {
     resid_part_body(L, F, save, pfix, blockIdx.x, gridDim.x);
 }
 __global__ void __launch_bounds__(256) k_resid_part_z(ZoneGrid G, int save) {
     const ZoneBlock b = zone_block(G);
-    resid_part_body(G.z[b.z].lv[1], G.z[b.z].F, save, 0, b.bid, b.nblk);
+    const Level L = G.z[b.z].lv[1];
+    const Fields F = G.z[b.z].F;
+    resid_part_body(L, F, save, 0, b.bid, b.nblk);
 }
 // one workgroup per zone
 __global__ void __launch_bounds__(256) k_resid_final_z(const ZoneDesc* __restrict__ z, int nblocks) {

@@ -542,7 +542,10 @@ __global__ void __launch_bounds__(256) k_prep(Level L, Fields F, Consts C, int m
 __global__ void __launch_bounds__(256) k_prep_z(ZoneGrid G, int n, int ucn_kept) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    prep_body(Z.lv[n], Z.F, Z.C, prep_mode(Z.C, n, ucn_kept), b.bid, b.nblk);
+    const Level L = Z.lv[n];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    prep_body(L, F, C, prep_mode(C, n, ucn_kept), b.bid, b.nblk);
 }
 __global__ void __launch_bounds__(256) k_residual(Level L, Fields F, Consts C, int n, int recalc) {
     residual_body(L, F, C, n, recalc, blockIdx.x, gridDim.x);
@@ -550,7 +553,10 @@ __global__ void __launch_bounds__(256) k_residual(Level L, Fields F, Consts C, i
 __global__ void __launch_bounds__(256) k_residual_z(ZoneGrid G, int n, int recalc) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    residual_body(Z.lv[n], Z.F, Z.C, n, recalc, b.bid, b.nblk);
+    const Level L = Z.lv[n];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    residual_body(L, F, C, n, recalc, b.bid, b.nblk);
 }
 __global__ void __launch_bounds__(kTX * kTY, 2) k_visc_pk(Level L, Fields F, Consts C, int n, int calc_pk, int kc) {
     visc_pk_body(L, F, C, n, calc_pk, kc, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
@@ -559,7 +565,10 @@ __global__ void __launch_bounds__(kTX * kTY, 2) k_visc_pk(Level L, Fields F, Con
 __global__ void __launch_bounds__(kTX * kTY, 2) k_visc_pk_z(ZoneGrid G, int n, int calc_pk, int kc) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    visc_pk_body(Z.lv[n], Z.F, Z.C, n, calc_pk, kc, b.bid, b.nblk);
+    const Level L = Z.lv[n];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    visc_pk_body(L, F, C, n, calc_pk, kc, b.bid, b.nblk);
 }
 
 }  // namespace
@@ -569,6 +578,11 @@ void launch_dtau(hipStream_t s, const Level& L, const Fields& F, const Consts& C
     hipLaunchKernelGGL(k_prep, dim3((unsigned)((L.n + b - 1) / b)), dim3(b), 0, s, L, F, C,
                        prep_mode(C, n, ucn_kept));
 }
+
+// tiles of all interior planes of a level
+static long visc_plane_tiles(const Level& L) { return (long)visc_gx(L) * visc_gy(L) * (L.nk - 2); }
+
+int visc_kc_default(const Level& L) { return kc_of_tiles(visc_plane_tiles(L)); }
 
 static unsigned node_blocks(const Level& L) { return (unsigned)((L.n + 255) / 256); }
 
@@ -582,10 +596,14 @@ void launch_residual_z(hipStream_t s, const ZoneList& Z, int n, int recalc, int 
     unsigned nb = 0;
     const ZoneGrid G = Z.grid([&](const ZoneDesc& z) { return node_blocks(z.lv[n]); }, nb);
     hipLaunchKernelGGL(k_residual_z, dim3(nb), dim3(256), 0, s, G, n, recalc);
-    // one plane count for every zone: the smallest zone's default
+    // one plane count for every zone, from the tiles of all of them: the
+    // launch fills the chip as a whole.  (The smallest zone's own default is
+    // one plane, whose two halo planes cost every zone: six blocks of 0.16 to
+    // 1.3 M nodes, 382 us at one plane, 250 us at nine.)
     if (kc <= 0) {
-        kc = 16;
-        for (const ZoneDesc& z : Z.host) kc = std::min(kc, visc_kc_default(z.lv[n]));
+        long t = 0;
+        for (const ZoneDesc& z : Z.host) t += visc_plane_tiles(z.lv[n]);
+        kc = kc_of_tiles(t);
     }
     for (const ZoneDesc& z : Z.host) kc = std::min(kc, z.lv[n].nk - 2);
     unsigned nv = 0;
@@ -593,12 +611,6 @@ void launch_residual_z(hipStream_t s, const ZoneList& Z, int n, int recalc, int 
         [&](const ZoneDesc& z) { return visc_gx(z.lv[n]) * visc_gy(z.lv[n]) * (unsigned)((z.lv[n].nk - 2 + kc - 1) / kc); },
         nv);
     hipLaunchKernelGGL(k_visc_pk_z, dim3(nv), dim3(kTX * kTY), 0, s, V, n, recalc ? 0 : calc_pk, kc);
-}
-
-int visc_kc_default(const Level& L) {
-    // planes per workgroup: enough workgroups (about 2048) to fill the chip
-    const long tiles = (long)((L.ni - 2 + kTX - 2) / (kTX - 1)) * ((L.nj - 2 + kTY - 2) / (kTY - 1));
-    return (int)std::max(1L, std::min(16L, tiles * (L.nk - 2) / 2048));
 }
 
 void launch_visc_pk(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int n, int calc_pk, int kc) {

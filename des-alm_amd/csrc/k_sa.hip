@@ -585,7 +585,9 @@ __device__ __forceinline__ void sa_sweep_body(const Level& L, const Fields& F, c
 __global__ void __launch_bounds__(256) k_sa_prep(Level L, Fields F) { sa_prep_body(L, F, blockIdx.x, gridDim.x); }
 __global__ void __launch_bounds__(256) k_sa_prep_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
-    sa_prep_body(G.z[b.z].lv[1], G.z[b.z].F, b.bid, b.nblk);
+    const Level L = G.z[b.z].lv[1];
+    const Fields F = G.z[b.z].F;
+    sa_prep_body(L, F, b.bid, b.nblk);
 }
 // three waves per SIMD: fits in 168 VGPRs without spilling
 __global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs(Level L, Fields F, Consts C, int kc) {
@@ -595,7 +597,10 @@ __global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs(Level L, Fields F, Cons
 __global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs_z(ZoneGrid G, int kc) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    sa_rhs_body(Z.lv[1], Z.F, Z.C, kc, b.bid, b.nblk);
+    const Level L = Z.lv[1];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    sa_rhs_body(L, F, C, kc, b.bid, b.nblk);
 }
 template <int D>
 __global__ void __launch_bounds__(256) k_sa_bc(Level L, Fields F, Consts C) {
@@ -605,13 +610,19 @@ template <int D>
 __global__ void __launch_bounds__(256) k_sa_bc_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    sa_bc_body<D>(Z.lv[1], Z.F, Z.C, b.bid);
+    const Level L = Z.lv[1];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    sa_bc_body<D>(L, F, C, b.bid);
 }
 __global__ void __launch_bounds__(256) k_sa_clamp(Level L, Fields F, Consts C) { sa_clamp_body(L, F, C, blockIdx.x); }
 __global__ void __launch_bounds__(256) k_sa_clamp_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    sa_clamp_body(Z.lv[1], Z.F, Z.C, b.bid);
+    const Level L = Z.lv[1];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    sa_clamp_body(L, F, C, b.bid);
 }
 template <int D, int R>
 __global__ void __launch_bounds__(512) k_sa_sweep(Level L, Fields F, Consts C, SegShape sh) {
@@ -621,15 +632,17 @@ template <int D, int R>
 __global__ void __launch_bounds__(512) k_sa_sweep_z(ZoneGrid G, int P, int TI) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    sa_sweep_body<D, R>(Z.lv[1], Z.F, Z.C, seg_lines(Z.lv[1], D, P, TI), xcd_block(b.bid, b.nblk));
+    const Level L = Z.lv[1];
+    const Fields F = Z.F;
+    const Consts C = Z.C;
+    sa_sweep_body<D, R>(L, F, C, seg_lines(L, D, P, TI), xcd_block(b.bid, b.nblk));
 }
 
 }  // namespace
 
-int sa_kc_default(const Level& L) {
-    const long tiles = (long)((L.ni - 2 + kQX - 2) / (kQX - 1)) * ((L.nj - 2 + kQY - 2) / (kQY - 1));
-    return (int)std::max(1L, std::min(16L, tiles * (L.nk - 2) / 2048));
-}
+static long sa_plane_tiles(const Level& L) { return (long)sa_gx(L) * sa_gy(L) * (L.nk - 2); }
+
+int sa_kc_default(const Level& L) { return kc_of_tiles(sa_plane_tiles(L)); }
 
 void launch_sa_prep(hipStream_t s, const Level& L, const Fields& F) {
     const int b = 256;
@@ -710,9 +723,12 @@ void launch_des_eddy_z(hipStream_t s, const ZoneList& Z, int itk, int kc) {
     const ZoneGrid Gi = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].nj * z.lv[1].nk + b - 1) / b); }, fi);
     const ZoneGrid Gj = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].ni * z.lv[1].nk + b - 1) / b); }, fj);
     const ZoneGrid Gk = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].ni * z.lv[1].nj + b - 1) / b); }, fk);
+    // one plane count from the tiles of all zones (as k_visc_pk's: 502 us at
+    // the one plane of the smallest of six blocks' own default, 400 us at nine)
     if (kc <= 0) {
-        kc = 16;
-        for (const ZoneDesc& z : Z.host) kc = std::min(kc, sa_kc_default(z.lv[1]));
+        long t = 0;
+        for (const ZoneDesc& z : Z.host) t += sa_plane_tiles(z.lv[1]);
+        kc = kc_of_tiles(t);
     }
     for (const ZoneDesc& z : Z.host) kc = std::min(kc, z.lv[1].nk - 2);
     const ZoneGrid Gq = Z.grid(
