@@ -44,6 +44,43 @@ __device__ __forceinline__ void st32(T* a, unsigned idx, T v) {
     *reinterpret_cast<T*>(reinterpret_cast<char*>(a) + idx * (unsigned)sizeof(T)) = v;
 }
 
+// FP64 division, reciprocal, reciprocal square root and square root from the
+// hardware estimates, for normal operands (a zero divisor or an infinite
+// operand gives NaN, a zero radicand an infinite reciprocal root and a zero
+// root).  One Newton step takes the ~2^-23 reciprocal estimate to ~2^-46 and
+// the residual step of the quotient, or a second Newton step, leaves about the
+// final rounding alone; the root's third-order step goes there at once.  Half
+// the instructions of the IEEE sequences, which also scale and fix up every
+// special case.
+__device__ __forceinline__ double div64(double a, double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+__device__ __forceinline__ double rcp64(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    return fma(r, fma(-b, r, 1.0), r);
+}
+__device__ __forceinline__ double rsqrt64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    const double r = fma(y * e, fma(0.375, e, 0.5), y);
+    return x == 0.0 ? y : r;
+}
+// sqrt(x) given y = rsqrt64(x)
+__device__ __forceinline__ double sqrt64(double x, double y) {
+    const double s = x * y;
+    const double r = fma(fma(-s, s, x), 0.5 * y, s);
+    return x == 0.0 ? 0.0 : r;
+}
+// 1 / x in the type of a line solve
+__device__ __forceinline__ double recip(double x) { return rcp64(x); }
+__device__ __forceinline__ float recip(float x) { return 1.0f / x; }
+__device__ __forceinline__ double quot(double a, double b) { return div64(a, b); }
+__device__ __forceinline__ float quot(float a, float b) { return a / b; }
+
 struct Level {
     int ni, nj, nk;
     long off;   // node offset of the level in all-level arrays

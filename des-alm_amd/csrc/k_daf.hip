@@ -43,15 +43,45 @@ namespace {
 // dtau-dependent factors of a node: sigma = sqrt(beta alpha) with
 // alpha = 1 + e_source 1.5 dtau / delti, and theta = sqrt(beta / alpha) =
 // beta / sigma (rhs_modal_matrices.F90:82-84)
+//
+// The FP64 form takes reciprocals and roots from the hardware estimates
+// (rcp64 and its like; errors of 0.5 ulp, 1 ulp for the reciprocal root, as
+// the IEEE operations they stand for).  The sweeps spent up to half their time
+// issuing instructions, two fifths of them divisions and roots: with these and
+// the scaling of maps and the divisions of the c' scan moved out of its serial
+// chain, i 124 -> 110 us, j 120 -> 109 us, k 150 -> 142 us on 193x129x129 and
+// 15.7 -> 12.4 us for the k sweep of 49x33x33, where the chain is all there is.
+// The FP32 form keeps the IEEE operations: its solves amplify any difference
+// of the transformed rows (one ulp of FP64 changes which FP32 value a row
+// rounds to), so its results would move by 1e-9 with nothing gained.
+template <typename S>
+struct Num {  // S = double
+    static __device__ __forceinline__ double rcp(double x) { return rcp64(x); }
+    // sqrt(x) and 1 / sqrt(x)
+    static __device__ __forceinline__ void root(double x, double& s, double& is) {
+        is = rsqrt64(x);
+        s = sqrt64(x, is);
+    }
+};
+template <>
+struct Num<float> {
+    static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+    static __device__ __forceinline__ void root(double x, double& s, double& is) {
+        s = sqrt(x);
+        is = 1.0 / s;
+    }
+};
+
 struct NodeDt {
     double dt, alpha, sigma, isigma, theta;
 };
+template <typename S>
 __device__ __forceinline__ NodeDt node_dt(const Consts& C, double dt) {
     NodeDt n;
     n.dt = dt;
-    n.alpha = 1.0 + C.e_source * 1.5 * dt / C.delti;
-    n.sigma = sqrt(C.beta * n.alpha);
-    n.isigma = 1.0 / n.sigma;
+    if (sizeof(S) == 8) n.alpha = 1.0 + C.e_source * 1.5 / C.delti * dt;
+    else n.alpha = 1.0 + C.e_source * 1.5 * dt / C.delti;
+    Num<S>::root(C.beta * n.alpha, n.sigma, n.isigma);
     n.theta = C.beta * n.isigma;
     return n;
 }
@@ -59,10 +89,12 @@ __device__ __forceinline__ NodeDt node_dt(const Consts& C, double dt) {
 // v <- M v for the Ma-type matrix of metric row (m1, m2, m3):
 //   row 0 = (0, 0, sigma, sigma); rows 1-3 = (t1/s, t2/(s sg), m/sg, -m/sg)
 //   with sg = |m|, s = sqrt(2 |m|^2 + (m2 - m3)^2)
+template <typename S>
 __device__ __forceinline__ void mul_m(double m1, double m2, double m3, double sigma, double v[4]) {
     const double g = m1 * m1 + m2 * m2 + m3 * m3;
-    const double isg = 1.0 / sqrt(g);
-    const double is = 1.0 / sqrt(2.0 * g + (m2 - m3) * (m2 - m3));
+    double sg, isg, s, is;
+    Num<S>::root(g, sg, isg);
+    Num<S>::root(2.0 * g + (m2 - m3) * (m2 - m3), s, is);
     const double w0 = v[0] * is, w1 = v[1] * (is * isg), u = (v[2] - v[3]) * isg;
     const double dm = m3 - m2;
     const double o0 = sigma * (v[2] + v[3]);
@@ -72,14 +104,15 @@ __device__ __forceinline__ void mul_m(double m1, double m2, double m3, double si
     v[0] = o0; v[1] = o1; v[2] = o2; v[3] = o3;
 }
 
-// v <- M^-1 v for the same matrix, given g = |m|^2 and sg = |m| (the inverse
-// in closed form, d = |m|^2 + 2 m2 m3 + m1^2)
-__device__ __forceinline__ void mul_minv(double m1, double m2, double m3, double g, double sg, double isigma,
+// v <- M^-1 v for the same matrix, given g = |m|^2 and isg = 1 / |m| (the
+// inverse in closed form, d = |m|^2 + 2 m2 m3 + m1^2)
+template <typename S>
+__device__ __forceinline__ void mul_minv(double m1, double m2, double m3, double g, double isg, double isigma,
                                          double v[4]) {
     const double m1s = m1 * m1, m2s = m2 * m2, m3s = m3 * m3;
-    const double s = sqrt(2.0 * g + (m2 - m3) * (m2 - m3));
-    const double id = 1.0 / (g + 2.0 * m2 * m3 + m1s);
-    const double isg = 1.0 / sg;
+    double s, is;
+    Num<S>::root(2.0 * g + (m2 - m3) * (m2 - m3), s, is);
+    const double id = Num<S>::rcp(g + 2.0 * m2 * m3 + m1s);
     const double r1 = m2 + m3, r2 = m2 - m3, r3 = m2s - m3s;
     const double o0 = s * id * (m1 * (v[2] + v[3]) - r1 * v[1]);
     const double o1 = s * isg * id *
@@ -91,19 +124,21 @@ __device__ __forceinline__ void mul_minv(double m1, double m2, double m3, double
     v[0] = o0; v[1] = o1; v[2] = t + p; v[3] = t - p;
 }
 
-// S (-dtau J rh) at global node g (rhs_diag_solver.F90:56-72): beta on the
-// pressure row, 1 / alpha on the velocity rows
+// S (-dtau J rh) (rhs_diag_solver.F90:56-72): beta on the pressure row,
+// 1 / alpha on the velocity rows
+template <typename S>
 __device__ __forceinline__ void scaled_rh_vals(const Consts& C, double aj, const double rh[4], const NodeDt& nd,
                                                double v[4]) {
     const double f = -nd.dt * aj;
-    const double ia = 1.0 / nd.alpha;
+    const double ia = Num<S>::rcp(nd.alpha);
     v[0] = C.beta * (f * rh[0]);
 #pragma unroll
     for (int m = 1; m < 4; m++) v[m] = ia * (f * rh[m]);
 }
+template <typename S>
 __device__ __forceinline__ void scaled_rh(const Fields& F, const Consts& C, long g, const NodeDt& nd, double v[4]) {
     const double rh[4] = {F.rh[0][g], F.rh[1][g], F.rh[2][g], F.rh[3][g]};
-    scaled_rh_vals(C, F.aj[g], rh, nd, v);
+    scaled_rh_vals<S>(C, F.aj[g], rh, nd, v);
 }
 
 // the metric row of direction D at node g
@@ -113,72 +148,59 @@ __device__ __forceinline__ void metric_row(const Fields& F, long g, double& m1, 
     m1 = mt[0][g]; m2 = mt[1][g]; m3 = mt[2][g];
 }
 
-// The modal transform that precedes sweep D at node g, applied to v
-// (Ma^-1; N1^-1 = Mb^-1 Ma; N2^-1 = Mc^-1 Mb, applied factor by factor),
-// and dtau times the spectral radius of direction D at g,
-// dtau theta |grad xi_D| (rhs_diag_solver.F90:149-160).
-// D = 0 builds its input S (-dtau J rh) here; D = 1, 2 take v as given.
-template <int D>
+// The modal transform that precedes sweep D (Ma^-1; N1^-1 = Mb^-1 Ma; N2^-1 =
+// Mc^-1 Mb, applied factor by factor) of v at a node, from values already
+// loaded: its dtau, the metric row a of direction D - 1 (unused for D = 0,
+// whose v is S (-dtau J rh)) and the row m of D.  Returns dtau times the
+// spectral radius of direction D, dtau theta |grad xi_D|
+// (rhs_diag_solver.F90:149-160).
+template <int D, typename S>
+__device__ __forceinline__ double transform_vals(const NodeDt& nd, const double a[3], const double m[3], double v[4]) {
+    if (D > 0) mul_m<S>(a[0], a[1], a[2], nd.sigma, v);
+    const double g = m[0] * m[0] + m[1] * m[1] + m[2] * m[2];
+    double sg, isg;
+    Num<S>::root(g, sg, isg);
+    mul_minv<S>(m[0], m[1], m[2], g, isg, nd.isigma, v);
+    return nd.dt * (nd.theta * sg);
+}
+template <typename S>
+__device__ __forceinline__ double sd_vals(const NodeDt& nd, const double m[3]) {
+    double sg, isg;
+    Num<S>::root(m[0] * m[0] + m[1] * m[1] + m[2] * m[2], sg, isg);
+    return nd.dt * (nd.theta * sg);
+}
+
+template <int D, typename S>
 __device__ __forceinline__ double transform_row(const Fields& F, const Consts& C, long g, double v[4]) {
-    const NodeDt nd = node_dt(C, F.dtau[g]);
-    if (D == 0) scaled_rh(F, C, g, nd, v);
-    if (D > 0) {
-        double a1, a2, a3;
-        metric_row<D - 1>(F, g, a1, a2, a3);
-        mul_m(a1, a2, a3, nd.sigma, v);
-    }
-    double m1, m2, m3;
-    metric_row<D>(F, g, m1, m2, m3);
-    const double gg = m1 * m1 + m2 * m2 + m3 * m3;
-    const double sg = sqrt(gg);
-    mul_minv(m1, m2, m3, gg, sg, nd.isigma, v);
-    return nd.dt * (nd.theta * sg);
+    const NodeDt nd = node_dt<S>(C, F.dtau[g]);
+    double a[3] = {0.0, 0.0, 0.0}, m[3];
+    if (D > 0) metric_row<(D > 0 ? D - 1 : 0)>(F, g, a[0], a[1], a[2]);
+    metric_row<D>(F, g, m[0], m[1], m[2]);
+    return transform_vals<D, S>(nd, a, m, v);
 }
-
-// the i sweep's transform (S then Ma^-1) and dtau spr from values already
-// loaded: dtau, J, rh and the csi row of one node
-__device__ __forceinline__ double transform_vals0(const Consts& C, double dt, double aj, const double rh[4], double m1,
-                                                  double m2, double m3, double v[4]) {
-    const NodeDt nd = node_dt(C, dt);
-    scaled_rh_vals(C, aj, rh, nd, v);
-    const double gg = m1 * m1 + m2 * m2 + m3 * m3;
-    const double sg = sqrt(gg);
-    mul_minv(m1, m2, m3, gg, sg, nd.isigma, v);
-    return nd.dt * (nd.theta * sg);
-}
-__device__ __forceinline__ double sd_vals(const Consts& C, double dt, double m1, double m2, double m3) {
-    const NodeDt nd = node_dt(C, dt);
-    return nd.dt * (nd.theta * sqrt(m1 * m1 + m2 * m2 + m3 * m3));
-}
-
-// dtau times the spectral radius of direction D alone
-template <int D>
+template <int D, typename S>
 __device__ __forceinline__ double row_sd(const Fields& F, const Consts& C, long g) {
-    const NodeDt nd = node_dt(C, F.dtau[g]);
-    double m1, m2, m3;
-    metric_row<D>(F, g, m1, m2, m3);
-    return nd.dt * (nd.theta * sqrt(m1 * m1 + m2 * m2 + m3 * m3));
+    const NodeDt nd = node_dt<S>(C, F.dtau[g]);
+    double m[3];
+    metric_row<D>(F, g, m[0], m[1], m[2]);
+    return sd_vals<S>(nd, m);
 }
 
 // the transform of sweep D alone (boundary vectors)
-template <int D>
+template <int D, typename S>
 __device__ __forceinline__ void pre_transform(const Fields& F, const Consts& C, long g, double v[4]) {
-    const NodeDt nd = node_dt(C, F.dtau[g]);
-    if (D > 0) {
-        double a1, a2, a3;
-        metric_row<D - 1>(F, g, a1, a2, a3);
-        mul_m(a1, a2, a3, nd.sigma, v);
-    }
-    double m1, m2, m3;
-    metric_row<D>(F, g, m1, m2, m3);
-    const double gg = m1 * m1 + m2 * m2 + m3 * m3;
-    mul_minv(m1, m2, m3, gg, sqrt(gg), nd.isigma, v);
+    const NodeDt nd = node_dt<S>(C, F.dtau[g]);
+    double a[3] = {0.0, 0.0, 0.0}, m[3];
+    if (D > 0) metric_row<(D > 0 ? D - 1 : 0)>(F, g, a[0], a[1], a[2]);
+    metric_row<D>(F, g, m[0], m[1], m[2]);
+    (void)transform_vals<D, S>(nd, a, m, v);
 }
 
 // v <- Mc v at global node g (rhs_diag_solver.F90:624-633)
+template <typename S>
 __device__ __forceinline__ void apply_mc(const Consts& C, double dtau, double z1, double z2, double z3, double v[4]) {
-    const NodeDt nd = node_dt(C, dtau);
-    mul_m(z1, z2, z3, nd.sigma, v);
+    const NodeDt nd = node_dt<S>(C, dtau);
+    mul_m<S>(z1, z2, z3, nd.sigma, v);
 }
 
 template <typename S>
@@ -235,6 +257,15 @@ __device__ __forceinline__ int pow2_exponent(S mx) {
     (void)frexp(mx, &e);
     return e;
 }
+template <typename S>
+__device__ __forceinline__ void scale_map(S (&m)[4]) {
+    const int e = -pow2_exponent(fmax(fmax(fabs(m[0]), fabs(m[1])), fmax(fabs(m[2]), fabs(m[3]))));
+#pragma unroll
+    for (int k = 0; k < 4; k++) m[k] = ldexp(m[k], e);
+}
+// rows composed between two scalings of a segment's map
+template <typename S>
+constexpr int kScaleRows = sizeof(S) == 8 ? 4 : 2;
 
 // One direction's DAF line solves on level L.
 //   D = 0: rows i = 1 .. ni-2 (+ the outlet plane when ext) of every (j, k)
@@ -286,6 +317,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
     // window entry w is node position s0 + w (row s0 + w - 1)
     S dv[R][4];
     S sdv[R + 2];
+    const int pe = s0 + nr + 1;  // the node after the segment
     if (D == 0) {
         // i lines: a segment's rows and its two window nodes are one run of
         // consecutive nodes, loaded as such (16-byte loads; lanes are R rows
@@ -312,18 +344,20 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
         double sdw[R + 2];
 #pragma unroll
         for (int w = 0; w < R + 2; w++) {
+            const NodeDt nd0 = node_dt<S>(C, dt[w]);
+            const double mr[3] = {m1[w], m2[w], m3[w]};
             if (w >= 1 && w <= R) {
                 const double rv[4] = {rh[0][w - 1], rh[1][w - 1], rh[2][w - 1], rh[3][w - 1]};
                 double v[4];
-                sdw[w] = transform_vals0(C, dt[w], aj[w - 1], rv, m1[w], m2[w], m3[w], v);
+                scaled_rh_vals<S>(C, aj[w - 1], rv, nd0, v);
+                sdw[w] = transform_vals<0, S>(nd0, mr, mr, v);
                 const bool in = w - 1 < nr;
 #pragma unroll
                 for (int m = 0; m < 4; m++) dv[w - 1][m] = in ? (S)v[m] : S(0);
             } else {
-                sdw[w] = sd_vals(C, dt[w], m1[w], m2[w], m3[w]);
+                sdw[w] = sd_vals<S>(nd0, mr);
             }
         }
-        const int pe = s0 + nr + 1;
         sdv[0] = nr > 0 ? (S)sdw[0] : S(0);
 #pragma unroll
         for (int w = 1; w <= R + 1; w++) {
@@ -332,9 +366,9 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
             const bool after = w == nr + 1 && nr > 0 && pe <= nd - 1;
             sdv[w] = (row || after) ? (S)sdw[w] : S(0);
         }
-    } else {
-        // j and k lines: one branch per row (all their rows' loads in flight
-        // would not fit the registers)
+    } else if (sizeof(S) == 4) {
+        // FP32: one branch per row, 125 and 146 VGPRs and three waves per
+        // SIMD (loaded ahead as below, 208 VGPRs and two waves, no faster)
 #pragma unroll
         for (int r = 0; r < R; r++) {
             sdv[r + 1] = S(0);
@@ -346,18 +380,54 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                 const long tl = base + (long)p * sD;
 #pragma unroll
                 for (int m = 0; m < 4; m++) v[m] = (double)io.xin[m][tl];
-                sdv[r + 1] = (S)transform_row<D>(F, C, gnode(p), v);
+                sdv[r + 1] = (S)transform_row<D, S>(F, C, gnode(p), v);
 #pragma unroll
                 for (int m = 0; m < 4; m++) dv[r][m] = (S)v[m];
             }
         }
-        const int pe = s0 + nr + 1;
-        sdv[0] = nr > 0 ? (S)row_sd<D>(F, C, gnode(s0)) : S(0);
-        const S se = (nr > 0 && pe <= nd - 1) ? (S)row_sd<D>(F, C, gnode(pe)) : S(0);
+        sdv[0] = nr > 0 ? (S)row_sd<D, S>(F, C, gnode(s0)) : S(0);
+        const S se = (nr > 0 && pe <= nd - 1) ? (S)row_sd<D, S>(F, C, gnode(pe)) : S(0);
         sdv[R + 1] = S(0);
 #pragma unroll
         for (int w = 1; w <= R + 1; w++)
             if (w == nr + 1) sdv[w] = se;
+    } else {
+        // j and k lines: the loads of window entry w + 1 are in flight while
+        // entry w is transformed, at addresses clamped to the line (no branch,
+        // which would hold back the next row's loads; all rows' loads at once
+        // would not fit the registers)
+        struct In {
+            double dt, a[3], m[3], x[4];
+        };
+        auto load = [&](int w, In& o) {
+            const long tl = base + (long)min(s0 + w, nd - 1) * sD, g = L.off + tl;
+            o.dt = F.dtau[g];
+            metric_row<D>(F, g, o.m[0], o.m[1], o.m[2]);
+            if (w >= 1 && w <= R) {
+                metric_row<(D > 0 ? D - 1 : 0)>(F, g, o.a[0], o.a[1], o.a[2]);
+#pragma unroll
+                for (int m = 0; m < 4; m++) o.x[m] = (double)io.xin[m][tl];
+            }
+        };
+        In cur, nxt;
+        load(0, cur);
+#pragma unroll
+        for (int w = 0; w < R + 2; w++) {
+            if (w + 1 < R + 2) load(w + 1, nxt);
+            const NodeDt nd0 = node_dt<S>(C, cur.dt);
+            if (w >= 1 && w <= R) {
+                const bool in = w - 1 < nr;
+                double v[4] = {cur.x[0], cur.x[1], cur.x[2], cur.x[3]};
+                const double sd = transform_vals<D, S>(nd0, cur.a, cur.m, v);
+                sdv[w] = (in || (w == nr + 1 && nr > 0)) ? (S)sd : S(0);
+#pragma unroll
+                for (int m = 0; m < 4; m++) dv[w - 1][m] = in ? (S)v[m] : S(0);
+            } else {
+                const double sd = sd_vals<S>(nd0, cur.m);
+                sdv[w] = (w == 0 ? nr > 0 : nr == R) ? (S)sd : S(0);
+            }
+            cur = nxt;
+        }
     }
     // semi-explicit boundary vectors of the first and last rows
     const bool first = act && s0 == 0 && nr > 0;
@@ -368,8 +438,8 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
         if (D == 0) {
             double r1[4], r2[4];
             const long g1 = gnode(1), g2 = gnode(2);
-            scaled_rh(F, C, g1, node_dt(C, F.dtau[g1]), r1);
-            scaled_rh(F, C, g2, node_dt(C, F.dtau[g2]), r2);
+            scaled_rh<S>(F, C, g1, node_dt<S>(C, F.dtau[g1]), r1);
+            scaled_rh<S>(F, C, g2, node_dt<S>(C, F.dtau[g2]), r2);
 #pragma unroll
             for (int m = 0; m < 4; m++) w[m] = C.sa[b0][m] * r1[m] + C.sb[b0][m] * r2[m];
         } else {
@@ -377,7 +447,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
             for (int m = 0; m < 4; m++)
                 w[m] = C.sa[b0][m] * (double)io.xin[m][base + sD] + C.sb[b0][m] * (double)io.xin[m][base + 2 * sD];
         }
-        pre_transform<D>(F, C, gnode(0), w);
+        pre_transform<D, S>(F, C, gnode(0), w);
 #pragma unroll
         for (int m = 0; m < 4; m++) {
             S am, bm, cm;
@@ -404,7 +474,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
             for (int m = 0; m < 4; m++)
                 w[m] = C.sa[b1][m] * (double)io.xin[m][base + (long)(nd - 2) * sD] +
                        C.sb[b1][m] * (double)io.xin[m][base + (long)(nd - 3) * sD];
-            pre_transform<D>(F, C, gnode(nd - 1), w);
+            pre_transform<D, S>(F, C, gnode(nd - 1), w);
         } else if (use_b1) {
             // brh(:,2) is not rebuilt when btype(6) == 6 (:467) and keeps
             // the fifth product of the k = 1 build (:462), which reads rh(1)
@@ -414,7 +484,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
             const double x1 = on_line ? (double)io.xin[0][base + sD + 1] : 0.0;
             const double x2 = on_line ? (double)io.xin[0][base + 2 * sD + 1] : 0.0;
             w[0] = C.sa[4][4] * x1 + C.sb[4][4] * x2;
-            pre_transform<D>(F, C, gnode(nd - 1), w);
+            pre_transform<D, S>(F, C, gnode(nd - 1), w);
         }
         const int r = nr - 1;
 #pragma unroll
@@ -455,10 +525,14 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                     // [c'; 1] -> [c; b - a c']
                     const S n0 = c * M[mi][2], n1 = c * M[mi][3];
                     const S n2 = b * M[mi][2] - a * M[mi][0], n3 = b * M[mi][3] - a * M[mi][1];
-                    const int e = -pow2_exponent(fmax(fmax(fabs(n0), fabs(n1)), fmax(fabs(n2), fabs(n3))));
-                    M[mi][0] = ldexp(n0, e); M[mi][1] = ldexp(n1, e); M[mi][2] = ldexp(n2, e); M[mi][3] = ldexp(n3, e);
+                    M[mi][0] = n0; M[mi][1] = n1; M[mi][2] = n2; M[mi][3] = n3;
                 }
             }
+            // scaled every few rows: exact, and the entries grow by no more
+            // than |a| + |b| + |c| per row (2 rows of FP32: up to 1e19 each)
+            if (r % kScaleRows<S> == kScaleRows<S> - 1 || r == R - 1)
+#pragma unroll
+                for (int mi = 0; mi < 3; mi++) scale_map(M[mi]);
         }
 #pragma unroll
         for (int mi = 0; mi < 3; mi++)
@@ -479,19 +553,23 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 if (sg0 + u < P) {
-                    sline[(sg0 + u) * kSlot + 4 * sm] = cn / cd;
+                    // the pair itself: every segment's thread divides for its own
+                    sline[(sg0 + u) * kSlot + 4 * sm] = cn;
+                    sline[(sg0 + u) * kSlot + 4 * sm + 1] = cd;
                     const S nn = q[u][0] * cn + q[u][1] * cd, dd = q[u][2] * cn + q[u][3] * cd;
-                    const int e = -pow2_exponent(fmax(fabs(nn), fabs(dd)));
-                    cn = ldexp(nn, e);
-                    cd = ldexp(dd, e);
+                    cn = nn;
+                    cd = dd;
                 }
             }
+            const int e = -pow2_exponent(fmax(fabs(cn), fabs(cd)));
+            cn = ldexp(cn, e);
+            cd = ldexp(cd, e);
         }
     }
     __syncthreads();
     S cst[3];
 #pragma unroll
-    for (int mi = 0; mi < 3; mi++) cst[mi] = slot[4 * mi];
+    for (int mi = 0; mi < 3; mi++) cst[mi] = quot(slot[4 * mi], slot[4 * mi + 1]);
 
     // ---- phase B: exact c' over the rows (their 1 / den kept); affine maps of d', scanned ----
     S inv[R][3];
@@ -511,7 +589,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                     S a, b, c;
                     coef(r, mi, a, b, c);
                     const S den = b - a * cprev;
-                    const S iv = S(1) / den;
+                    const S iv = recip(den);
                     inv[r][mi] = iv;
                     cprev = c * iv;
                     if (!(den != S(0) && isfinite(den)) && zrow == 0) zrow = s0 + r + 1;
@@ -589,6 +667,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                     S a, b, c;
                     coef(r, mi, a, b, c);
                     const S cc = c * inv[r][mi];
+                    inv[r][mi] = cc;  // c' from here on
 #pragma unroll
                     for (int m = 0; m < 4; m++) {
                         if (mat_of(m) == mi) {
@@ -630,9 +709,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
         if (r < nr) {
 #pragma unroll
             for (int mi = 0; mi < 3; mi++) {
-                S a, b, c;
-                coef(r, mi, a, b, c);
-                const S cc = c * inv[r][mi];
+                const S cc = inv[r][mi];
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
                     if (mat_of(m) == mi) {
@@ -671,7 +748,7 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                 for (int m = 0; m < 4; m++) qv[u][m] = F.q[m][g];
 #pragma unroll
                 for (int m = 0; m < 4; m++) v[u][m] = (double)dv[r0 + u][m];
-                apply_mc(C, dt, z1, z2, z3, v[u]);
+                apply_mc<S>(C, dt, z1, z2, z3, v[u]);
 #pragma unroll
                 for (int m = 0; m < 4; m++) qv[u][m] = qv[u][m] + v[u][m];
             }

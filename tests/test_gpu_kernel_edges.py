@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import mlp_oracle as mo
+import pyoracle as po
 from desalm import cases
 from desalm.lib import Solver
 
@@ -63,4 +64,25 @@ def test_learned_start_tiles(gpu, nh, dims):
     assert (np.abs(got[g] - want[g]).max(axis=0) <= 2e-5 * scale + 1e-14).all()
     rest = np.setdiff1d(np.arange(len(q)), g)
     assert np.array_equal(got[rest], q[rest])
+    s.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("dims", [(5, 6, 7), (12, 67, 9), (9, 10, 68), (67, 11, 75), (18, 66, 67)])
+def test_line_sweep_segments(gpu, dims, prec):
+    """Lines of 3 to 73 rows: partial last segments, lines at the change from
+    four to eight rows per segment (64 rows), fewer lines than a workgroup
+    takes."""
+    c = cases.wavy(*dims, ng=1, itm=2, des=True, precision=prec)
+    s = Solver(c.params).load_case(c)
+    s.mg_driver()
+    q, _, _, x = s.get_state()
+    o = po.Oracle(c.params).load_case(c)
+    o.mg_driver()
+    qo, _, _, xo = o.get_state()
+    # FP64 sums of a few hundred terms; FP32 solves of dq as a defect correction
+    tol = 1e-6 if prec else 1e-10
+    assert max(po.relerr(q[:, m], qo[:, m]) for m in range(5)) <= tol
+    assert po.relerr(x, xo) <= tol
+    assert s.pivot_events == 0
     s.close()
