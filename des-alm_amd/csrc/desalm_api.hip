@@ -85,6 +85,9 @@ struct desalm_ctx {
     bool sizing = false;
     double* staging = nullptr;     // 5 * nall doubles: AoS transfers
     double* dq_buf = nullptr;      // 4 * n1 doubles: dq of the solver_daf parity entry
+    // pinned host memory: the update norms' L1 sums and the zero-pivot word, as
+    // the last kernel of a pseudo-iteration stores them (F.host_sums)
+    double* host_sums = nullptr;
     std::string err;
     double last_ms = 0.0;
     unsigned long long last_pivots = 0;
@@ -469,6 +472,9 @@ int desalm_init(const desalm_params* p, int device, desalm_ctx** out) {
     }
     fields();
     if (ok) F.zero_pivot = (unsigned*)(F.resid + 5);
+    if (hipHostMalloc((void**)&c->host_sums, 6 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer((void**)&F.host_sums, c->host_sums, 0) != hipSuccess)
+        ok = false;
     {
         void* pv = nullptr;
         if (hipMalloc(&pv, sizeof(unsigned long long)) != hipSuccess) ok = false;
@@ -732,8 +738,6 @@ static int vcycles(std::vector<desalm_ctx*>& zs, bool have_table, int apply_mom,
     HIPCHK(c0, hipGetLastError());
     const Level& L0 = c0->lv[1];
     const double tnu = (double)((long)(L0.ni - 2) * (L0.nj - 2) * (L0.nk - 2));
-    // per zone: the five L1 sums and the zero-pivot word (F.resid[0..5])
-    std::vector<double> parts(6 * zs.size());
     int itc = 0;
     int rc = 0;
     // decide_recalc_rh is carried from level to level and from one
@@ -763,10 +767,13 @@ static int vcycles(std::vector<desalm_ctx*>& zs, bool have_table, int apply_mom,
                     if (have_table) timed(c0, KID_OVERSET, 1, [&] { exchange(1); });
                 }
                 const bool ucn_kept = p.des && n == 1;
+                // the coarsest level's residual is restricted nowhere, and its
+                // next pass forms it anew: it is left to the end of the call
+                const int recalc = n == ng && ng > 1 ? 0 : decide_recalc_rh;
                 if (zl)
-                    solver_daf_zones(zs, *zl, n, decide_recalc_rh, itr, ucn_kept);
+                    solver_daf_zones(zs, *zl, n, recalc, itr, ucn_kept);
                 else
-                    for (desalm_ctx* c : zs) solver_daf(c, n, decide_recalc_rh, itr, nullptr, ucn_kept);
+                    for (desalm_ctx* c : zs) solver_daf(c, n, recalc, itr, nullptr, ucn_kept);
                 // wall functions on the j walls of zone 1 (mg_driver.F90:218-224)
                 if (n == 1 && (c0->hooks & DESALM_HOOK_WALL_FUNCTIONS))
                     timed(c0, KID_BCOND, 1, [&] { launch_wall_functions(s, c0->lv[1], c0->F, c0->p.ren); });
@@ -851,13 +858,11 @@ static int vcycles(std::vector<desalm_ctx*>& zs, bool have_table, int apply_mom,
             decide_recalc_rh = body(decide_recalc_rh);
         }
         HIPCHK(c0, hipGetLastError());
-        for (size_t z = 0; z < zs.size(); z++)
-            HIPCHK(c0, hipMemcpyAsync(&parts[6 * z], zs[z]->F.resid, 6 * sizeof(double), hipMemcpyDeviceToHost, s));
         HIPCHK(c0, hipStreamSynchronize(s));
         for (desalm_ctx* c : zs) prof_flush(c);
         double resd[5] = {0, 0, 0, 0, 0};
         for (size_t z = 0; z < zs.size(); z++)
-            for (int m = 0; m < 5; m++) resd[m] = resd[m] + parts[6 * z + m];
+            for (int m = 0; m < 5; m++) resd[m] = resd[m] + zs[z]->host_sums[m];
         double residual[5];
         for (int m = 0; m < 5; m++) residual[m] = log10(resd[m] / tnu);
         if (resid_out)
@@ -869,7 +874,7 @@ static int vcycles(std::vector<desalm_ctx*>& zs, bool have_table, int apply_mom,
         unsigned zp = 0xffffffffu;
         for (size_t z = 0; z < zs.size(); z++) {
             unsigned w = 0;
-            memcpy(&w, &parts[6 * z + 5], sizeof(unsigned));
+            memcpy(&w, &zs[z]->host_sums[5], sizeof(unsigned));
             zp = std::min(zp, w);
         }
         bool nonfinite = false;
@@ -898,6 +903,18 @@ static int vcycles(std::vector<desalm_ctx*>& zs, bool have_table, int apply_mom,
         if (itc > p.it_min && ermax < p.er_min) converged = true;
         if (itc > p.it_min && eomax < p.eo_min) converged = true;
         if (converged) break;
+    }
+    // rh of the coarsest level as its last pass leaves it (solver_daf.F90:432-484):
+    // its q has not changed since.  Once per pass of every pseudo-iteration it
+    // took three launch pairs of about 16 us each on 49x33x33.
+    if (itc > 0 && ng > 1 && p.iter[ng - 1] > 0 && carried == 1) {
+        if (zl)
+            timed(c0, KID_RESIDUAL_RECALC, ng, [&] { launch_residual_z(s, *zl, ng, 1, 0, c0->kc_visc[ng]); });
+        else
+            for (desalm_ctx* c : zs)
+                timed(c, KID_RESIDUAL_RECALC, ng,
+                      [&] { launch_residual(s, c->lv[ng], c->F, c->C, ng, 1, 0, c->kc_visc[ng]); });
+        HIPCHK(c0, hipGetLastError());
     }
     for (desalm_ctx* c : zs)
         HIPCHK(c0, hipMemcpyAsync(&c->last_pivots, c->F.pivots, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
@@ -1645,7 +1662,7 @@ int desalm_autotune(desalm_ctx* c, int reps) {
         for (int kc : cand) {
             if (kc > L.nk - 2) break;
             float ms = 0.0f;
-            if (time_it([&] { launch_sa_rhs(s, L, c->F, c->C, kc); }, ms)) return -1;
+            if (time_it([&] { launch_sa_rhs(s, L, c->F, c->C, kc, false); }, ms)) return -1;
             if (ms < best) { best = ms; pick = kc; }
         }
         c->kc_sa = pick;
@@ -2023,6 +2040,7 @@ int desalm_finalize(desalm_ctx* c) {
     for (hipEvent_t e : c->prof.pool) (void)hipEventDestroy(e);
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->probe_dev) (void)hipFree(c->probe_dev);
+    if (c->host_sums) (void)hipHostFree(c->host_sums);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);

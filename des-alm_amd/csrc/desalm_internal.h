@@ -137,6 +137,7 @@ struct Fields {
     double* rh5;      // fine: SA right-hand side
     double* resid_part;  // [kResidBlocks * 5] partial L1 sums
     double* resid;       // [5] L1 sums
+    double* host_sums;   // [6] pinned host memory: the L1 sums and the zero-pivot word
     double* pfix;        // [1] pinned pressure value
     // inflow (btype 4) and characteristic-outlet (btype 5) faces of the i and
     // j directions: grid ratio of the extrapolation per face node (null where
@@ -146,7 +147,15 @@ struct Fields {
     unsigned* zero_pivot;        // [1] first line row with a zero or non-finite pivot (0xffffffff: none)
 };
 
+// workgroups of a norm over n nodes: one node per thread up to kResidBlocks
+// (33^3 nodes in 4096 workgroups took 7.8 us and their partial sums another
+// 6.5 us, in 140 workgroups 5.3 and 3.9 us; in 35 of four nodes per thread
+// 8.9 us, four memory latencies in turn)
 constexpr int kResidBlocks = 4096;
+__host__ __device__ inline int resid_blocks(long n) {
+    const long b = n / 256;
+    return (int)(b < 1 ? 1 : b > kResidBlocks ? kResidBlocks : b);
+}
 
 // Overset donor table of the fine level (device pointers, level-local node
 // indices): donor d reads the cell whose lower corner is host[d] with
@@ -331,7 +340,8 @@ void launch_bcond_fm(hipStream_t s, const Level& L, const Fields& F, const Const
 // SA / DES, k_sa.hip
 void launch_des_eddy(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int itk, int kc);
 void launch_sa_prep(hipStream_t s, const Level& L, const Fields& F);
-void launch_sa_rhs(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int kc);
+// floored: nu~ is read raised to its floor (a later sub-iteration of des_eddy)
+void launch_sa_rhs(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int kc, bool floored);
 int sa_kc_default(const Level& L);
 // multigrid, k_mg.hip
 void launch_inject(hipStream_t s, const Level* lv, int ng, int icrs, int jcrs, int kcrs,

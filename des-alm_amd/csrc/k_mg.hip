@@ -11,7 +11,7 @@
 //   k_rs_sweep<D>   rs_sweep constant-coefficient smoothing sweeps
 //                   (src/rs_sweep.F90:59-178) with every row on chip,
 //                   k sweep also adds dq to q
-//   k_bc_fm<D>      bcond_fm faces (src/bcond_fm.F90:79-306), k_pfix_*
+//   k_bc_fm         bcond_fm faces (src/bcond_fm.F90:79-306), k_pfix_*
 //                   the pinned-pressure shift (:310-322)
 //   k_resid_*       mg_residual's L1 update norms (src/mg_residual.F90:58-67)
 #include "desalm_internal.h"
@@ -24,6 +24,8 @@ namespace {
 __device__ __forceinline__ long lidx(const Level& L, int i, int j, int k) {
     return (long)i + (long)L.ni * ((long)j + (long)L.nj * k);
 }
+
+inline long lidx_h(const Level& L, int i, int j, int k) { return (long)i + (long)L.ni * ((long)j + (long)L.nj * k); }
 
 // coarse node (i,j,k) -> coincident fine node, 0-based (fine 1-based index
 // 2^crs * i - crs of src/mg_nlevel.F90:22-24)
@@ -340,105 +342,203 @@ __global__ void k_outlet_ratio(Level L, Fields F, int b, int dir) {
     F.rat[b][t] = (b % 2 == 0) ? (c1 - c0) / (c2 - c1) : (c0 - c1) / (c1 - c2);
 }
 
-// ---- bcond_fm faces of direction D (both sides) ----
+// ---- bcond_fm faces ----
+// The reference sets the i faces, then the j faces, then the k faces, each
+// over boundary nodes too, so an edge node reads face nodes of the direction
+// before.  One launch does all three: the value a node has after direction E
+// is formed from the values its one or two source nodes have after direction
+// E - 1, down to nodes that no face writes (bc_value), and a node is stored by
+// the thread of its last direction alone.  The nodes read from memory are
+// written by no thread: a source of direction E lies one or two nodes off that
+// face, and a source on a later direction's face belongs to a node that the
+// later direction overwrites.  (Three launches in sequence: 15 us on a level
+// of 33^3 nodes, where each is little more than its launch; 8.4 us in one.)
+// Exception: a plane copy (btype 6) on one face of a direction only reads the
+// opposite plane that its own rule overwrites; then every direction has its
+// own launch (E0 = E1), whose threads hold both faces of a line.
 // Inflow (btype 4) on a k face uses ratio 0: the reference fills its table
 // only where btype == 4 .and. btype == 5 (init.F90:2855, :2874), i.e. never,
 // and the table is zero as allocated.
-// the four components of q at node g; each face below loads all it reads
-// before its first store, so that the loads are in flight together
-__device__ __forceinline__ void load4(const Fields& F, long g, double v[4]) {
+template <int E0, int E>
+struct BcValue {
+    // q(1:4) after directions E0 .. E at node p
+    static __device__ __forceinline__ void get(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                               double (&v)[4]) {
+        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
+        if (p[E] == 0) low(L, F, C, p, v);
+        else if (p[E] == nd - 1) high(L, F, C, p, v);
+        else BcValue<E0, E - 1>::get(L, F, C, p, v);
+    }
+    static __device__ __forceinline__ void before(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                  int pos, double (&v)[4]) {
+        int s[3] = {p[0], p[1], p[2]};
+        s[E] = pos;
+        BcValue<E0, E - 1>::get(L, F, C, s, v);
+    }
+    // grid ratio of an inflow face at node p
+    static __device__ __forceinline__ double ratio(const Level& L, const Fields& F, int b, const int (&p)[3]) {
+        if (E == 2) return 0.0;
+        return E == 0 ? F.rat[b][p[1] + (long)L.nj * p[2]] : F.rat[b][p[0] + (long)L.ni * p[2]];
+    }
+    // the common rules of face b, node pos on it, s one node off it, s2 two
+    static __device__ __forceinline__ void face(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                int bt, int b, int pos, int s, int s2, double (&v)[4]) {
+        double a[4], c[4];
+        if (bt >= 1 && bt <= 3) {
+            before(L, F, C, p, s, a);
+            before(L, F, C, p, s2, c);
 #pragma unroll
-    for (int m = 0; m < 4; m++) v[m] = F.q[m][g];
+            for (int m = 0; m < 4; m++) v[m] = C.sa[b][m] * a[m] + C.sb[b][m] * c[m];
+        } else {
+            before(L, F, C, p, pos, v);
+            if (bt == 4) {  // inflow: pressure extrapolated on the grid ratio (bcond_fm.F90:95-102)
+                const double r = ratio(L, F, b, p);
+                before(L, F, C, p, s, a);
+                before(L, F, C, p, s2, c);
+                v[0] = (1.0 + r) * a[0] - r * c[0];
+            }
+        }
+    }
+    static __device__ __forceinline__ void low(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                               double (&v)[4]) {
+        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
+        const int bt = C.btype[2 * E];
+        // plane copy from the opposite boundary plane (not done for i);
+        // periodic wrap: the image of the opposite interior plane
+        if (bt == 6 && E > 0) before(L, F, C, p, nd - 1, v);
+        else if (bt == 7) before(L, F, C, p, nd - 2, v);
+        else face(L, F, C, p, bt, 2 * E, 0, 1, 2, v);
+    }
+    static __device__ __forceinline__ void high(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                double (&v)[4]) {
+        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
+        const int bt = C.btype[2 * E + 1];
+        if (bt == 6 && E > 0) low(L, F, C, p, v);  // the low plane as it is by now
+        else if (bt == 7) before(L, F, C, p, 1, v);
+        else if (bt == 8 && E == 0) before(L, F, C, p, nd - 2, v);
+        else face(L, F, C, p, bt, 2 * E + 1, nd - 1, nd - 2, nd - 3, v);
+    }
+};
+// before the first direction: memory
+template <int E0>
+struct BcBase {
+    static __device__ __forceinline__ void get(const Level& L, const Fields& F, const Consts&, const int (&p)[3],
+                                               double (&v)[4]) {
+        const long g = L.off + lidx(L, p[0], p[1], p[2]);
+#pragma unroll
+        for (int m = 0; m < 4; m++) v[m] = F.q[m][g];
+    }
+};
+template <>
+struct BcValue<0, -1> : BcBase<0> {};
+template <>
+struct BcValue<1, 0> : BcBase<1> {};
+template <>
+struct BcValue<2, 1> : BcBase<2> {};
+
+// workgroups of the faces of directions E0 .. E1 (a workgroup has one
+// direction); in one launch each side its own, then one for the pinned node
+__host__ __device__ inline unsigned face_blocks(const Level& L, int E) {
+    const long n = E == 0 ? (long)L.nj * L.nk : E == 1 ? (long)L.ni * L.nk : (long)L.ni * L.nj;
+    return (unsigned)((n + 255) / 256);
 }
-__device__ __forceinline__ void store4(const Fields& F, long g, const double v[4]) {
-#pragma unroll
-    for (int m = 0; m < 4; m++) F.q[m][g] = v[m];
+__host__ __device__ inline unsigned face_blocks(const Level& L, int E0, int E1) {
+    unsigned n = 0;
+    for (int e = E0; e <= E1; e++) n += face_blocks(L, e);
+    return E0 == E1 ? n : 2 * n + 1;
+}
+// line t of direction e: position of its low node; false past the last line
+__device__ __forceinline__ bool face_line(const Level& L, int e, long t, int (&p)[3]) {
+    const int n0 = e == 0 ? L.nj : L.ni, n1 = e == 2 ? L.nj : L.nk;
+    if (t >= (long)n0 * n1) return false;
+    const int a = (int)(t % n0), b = (int)(t / n0);
+    p[0] = e == 0 ? 0 : a;
+    p[1] = e == 0 ? a : e == 1 ? 0 : b;
+    p[2] = e == 2 ? 0 : b;
+    return true;
 }
 
-template <int D>
-__device__ __forceinline__ void bc_fm_body(const Level& L, const Fields& F, const Consts& C, unsigned bid) {
-    const int ni = L.ni, nj = L.nj, nk = L.nk;
-    const long sI = 1, sJ = ni, sK = (long)ni * nj;
-    const long t = (long)bid * blockDim.x + threadIdx.x;
-    long base, sD;
-    int nd;
-    if (D == 0) {
-        if (t >= (long)nj * nk) return;
-        base = sJ * (t % nj) + sK * (t / nj);
-        sD = sI;
-        nd = ni;
-    } else if (D == 1) {
-        if (t >= (long)ni * nk) return;
-        base = (t % ni) + sK * (t / ni);
-        sD = sJ;
-        nd = nj;
-    } else {
-        if (t >= (long)ni * nj) return;
-        base = t;
-        sD = sK;
-        nd = nk;
-    }
-    const long lo = L.off + base, hi = L.off + base + (long)(nd - 1) * sD;
-    const int b0 = 2 * D, b1 = 2 * D + 1;
+// side: 0 low face, 1 high face (one launch for all directions: adjacent
+// workgroups, so that an edge node's chain of reads is that of one side), 2
+// both
+template <int E0, int E, int E1>
+__device__ __forceinline__ void bc_store(const Level& L, const Fields& F, const Consts& C, int (&p)[3], int side,
+                                         long nfix) {
+    const int nd[3] = {L.ni, L.nj, L.nk};
+    // nodes on a later direction's face belong to its threads
+    for (int e = E + 1; e <= E1; e++)
+        if (p[e] == 0 || p[e] == nd[e] - 1) return;
     double a[4], b[4];
-    switch (C.btype[b0]) {
-        case 1: case 2: case 3:
-            load4(F, lo + sD, a);
-            load4(F, lo + 2 * sD, b);
+    if (side != 2) {
+        if (side) p[E] = nd[E] - 1;
+        BcValue<E0, E>::get(L, F, C, p, a);
+        const long g = L.off + lidx(L, p[0], p[1], p[2]);
 #pragma unroll
-            for (int m = 0; m < 4; m++) a[m] = C.sa[b0][m] * a[m] + C.sb[b0][m] * b[m];
-            store4(F, lo, a);
-            break;
-        case 6:  // plane copy from the opposite boundary plane (not done for i)
-            if (D > 0) {
-                load4(F, hi, a);
-                store4(F, lo, a);
-            }
-            break;
-        case 7:  // periodic wrap: the image of the opposite interior plane
-            load4(F, hi - sD, a);
-            store4(F, lo, a);
-            break;
-        case 4: {  // inflow: pressure extrapolated on the grid ratio (bcond_fm.F90:95-102)
-            const double r = D < 2 ? F.rat[b0][t] : 0.0;
-            F.q[0][lo] = (1.0 + r) * F.q[0][lo + sD] - r * F.q[0][lo + 2 * sD];
-            break;
-        }
-        default: break;
+        for (int m = 0; m < 4; m++) F.q[m][g] = a[m];
+        return;
     }
-    switch (C.btype[b1]) {
-        case 1: case 2: case 3:
-            load4(F, hi - sD, a);
-            load4(F, hi - 2 * sD, b);
+    BcValue<E0, E>::low(L, F, C, p, a);
+    const long lo = L.off + lidx(L, p[0], p[1], p[2]);
+    p[E] = nd[E] - 1;
+    BcValue<E0, E>::high(L, F, C, p, b);
+    const long hi = L.off + lidx(L, p[0], p[1], p[2]);
+    // one launch per direction: the pinned node's pressure comes from the
+    // thread of its k line, since a one-sided plane copy to it reads the plane
+    // that this line's other end overwrites
+    if (E == 2 && lo - L.off == nfix % ((long)L.ni * L.nj)) {
+        const long g = L.off + nfix;
+        *F.pfix = g == lo ? a[0] : g == hi ? b[0] : F.q[0][g];
+    }
 #pragma unroll
-            for (int m = 0; m < 4; m++) a[m] = C.sa[b1][m] * a[m] + C.sb[b1][m] * b[m];
-            store4(F, hi, a);
-            break;
-        case 6:
-            if (D > 0) {
-                load4(F, lo, a);
-                store4(F, hi, a);
-            }
-            break;
-        case 7:
-            load4(F, lo + sD, a);
-            store4(F, hi, a);
-            break;
-        case 4: {
-            const double r = D < 2 ? F.rat[b1][t] : 0.0;
-            F.q[0][hi] = (1.0 + r) * F.q[0][hi - sD] - r * F.q[0][hi - 2 * sD];
-            break;
-        }
-        case 8:
-            if (D == 0) {
-                load4(F, hi - sD, a);
-                store4(F, hi, a);
-            }
-            break;
-        default: break;
+    for (int m = 0; m < 4; m++) {
+        F.q[m][lo] = a[m];
+        F.q[m][hi] = b[m];
     }
 }
 
+// faces of directions E0 .. E1; with the last direction also the pressure of
+// the pinned node after it (bcond_fm.F90:310-322) into F.pfix
+template <int E0, int E1>
+__device__ __forceinline__ void bc_fm_body(const Level& L, const Fields& F, const Consts& C, long nfix, unsigned bid,
+                                           unsigned nblk) {
+    if (E0 != E1 && bid == nblk - 1) {
+        if (threadIdx.x != 0) return;
+        const int p[3] = {(int)(nfix % L.ni), (int)((nfix / L.ni) % L.nj), (int)(nfix / ((long)L.ni * L.nj))};
+        double v[4];
+        BcValue<E0, E1>::get(L, F, C, p, v);
+        *F.pfix = v[0];
+        return;
+    }
+    int p[3];
+    const int side = E0 == E1 ? 2 : (int)(bid & 1u);
+    unsigned b = E0 == E1 ? bid : bid >> 1;
+    if constexpr (E0 == 0) {
+        const unsigned n = face_blocks(L, 0);
+        if (b < n) {
+            if (face_line(L, 0, (long)b * 256 + threadIdx.x, p)) bc_store<E0, 0, E1>(L, F, C, p, side, nfix);
+            return;
+        }
+        b -= n;
+    }
+    if constexpr (E0 <= 1 && E1 >= 1) {
+        const unsigned n = face_blocks(L, 1);
+        if (b < n) {
+            if (face_line(L, 1, (long)b * 256 + threadIdx.x, p)) bc_store<E0, 1, E1>(L, F, C, p, side, nfix);
+            return;
+        }
+        b -= n;
+    }
+    if constexpr (E1 == 2) {
+        if (face_line(L, 2, (long)b * 256 + threadIdx.x, p)) bc_store<E0, 2, E1>(L, F, C, p, side, nfix);
+    }
+}
+
+// whether a direction copies planes on one face only
+inline bool one_sided_copy(const Consts& C) {
+    for (int e = 1; e < 3; e++)
+        if ((C.btype[2 * e] == 6) != (C.btype[2 * e + 1] == 6)) return true;
+    return false;
+}
 
 __device__ __forceinline__ void pfix_sub_body(const Level& L, const Fields& F, unsigned bid) {
     const long t = (long)bid * blockDim.x + threadIdx.x;
@@ -509,9 +609,16 @@ __device__ __forceinline__ void resid_final_body(const Fields& F, int nblocks) {
         }
         __syncthreads();
     }
+    // the sums stay on the device and go, with the zero-pivot word, straight
+    // to the host memory that the driver reads after the pseudo-iteration (a
+    // copy command of its own cost 4 us on the stream)
     if (threadIdx.x == 0) {
 #pragma unroll
-        for (int m = 0; m < 5; m++) F.resid[m] = sh[m][0];
+        for (int m = 0; m < 5; m++) {
+            F.resid[m] = sh[m][0];
+            F.host_sums[m] = sh[m][0];
+        }
+        *reinterpret_cast<unsigned*>(F.host_sums + 5) = *F.zero_pivot;
     }
 }
 
@@ -569,28 +676,18 @@ __global__ void __launch_bounds__(512) k_rs_sweep_z(ZoneGrid G, int n, int P, in
     const Fields F = Z.F;
     rs_sweep_body<D, R>(L, F, seg_lines(L, D, P, TI), Z.C.ep[1][D], xcd_block(b.bid, b.nblk));
 }
-// D = 2 also reads the pinned pressure into F.pfix (bcond_fm.F90:310-322),
-// in the thread of the pinned node's k column (face node tfix) after that
-// thread's own face writes: no other thread of the launch writes the
-// column, and the i and j faces are complete
-template <int D>
-__global__ void __launch_bounds__(256) k_bc_fm(Level L, Fields F, Consts C, long tfix, long gfix) {
-    bc_fm_body<D>(L, F, C, blockIdx.x);
-    if (D == 2 && (long)blockIdx.x * blockDim.x + threadIdx.x == tfix) *F.pfix = F.q[0][gfix];
+template <int E0, int E1>
+__global__ void __launch_bounds__(256) k_bc_fm(Level L, Fields F, Consts C, long nfix) {
+    bc_fm_body<E0, E1>(L, F, C, nfix, blockIdx.x, gridDim.x);
 }
-template <int D>
+template <int E0, int E1>
 __global__ void __launch_bounds__(256) k_bc_fm_z(ZoneGrid G) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
     const Level L = Z.lv[1];
     const Fields F = Z.F;
     const Consts C = Z.C;
-    bc_fm_body<D>(L, F, C, b.bid);
-}
-// one thread per zone
-__global__ void k_pfix_read_z(const ZoneDesc* __restrict__ z, int nz) {
-    const int t = (int)threadIdx.x;
-    if (t < nz) *z[t].F.pfix = z[t].F.q[0][z[t].pfix];
+    bc_fm_body<E0, E1>(L, F, C, Z.pfix - L.off, b.bid, b.nblk);
 }
 __global__ void __launch_bounds__(256) k_pfix_sub(Level L, Fields F) { pfix_sub_body(L, F, blockIdx.x); }
 __global__ void __launch_bounds__(256) k_pfix_sub_z(ZoneGrid G) {
@@ -609,8 +706,8 @@ __global__ void __launch_bounds__(256) k_resid_part_z(ZoneGrid G, int save) {
     resid_part_body(L, F, save, 0, b.bid, b.nblk);
 }
 // one workgroup per zone
-__global__ void __launch_bounds__(256) k_resid_final_z(const ZoneDesc* __restrict__ z, int nblocks) {
-    resid_final_body(z[blockIdx.x].F, nblocks);
+__global__ void __launch_bounds__(256) k_resid_final_z(const ZoneDesc* __restrict__ z) {
+    resid_final_body(z[blockIdx.x].F, resid_blocks(z[blockIdx.x].lv[1].n));
 }
 
 inline unsigned nblk(long n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -673,11 +770,14 @@ void launch_outlet_ratios(hipStream_t s, const Level& L, const Fields& F, const 
 
 void launch_bcond_fm(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int ifix, int jfix, int kfix,
                      bool pfix_deferred) {
-    const long tfix = (ifix - 1) + (long)L.ni * (jfix - 1);
-    const long g = L.off + tfix + (long)L.ni * L.nj * (kfix - 1);
-    hipLaunchKernelGGL(k_bc_fm<0>, dim3(nblk((long)L.nj * L.nk, 256)), dim3(256), 0, s, L, F, C, -1L, g);
-    hipLaunchKernelGGL(k_bc_fm<1>, dim3(nblk((long)L.ni * L.nk, 256)), dim3(256), 0, s, L, F, C, -1L, g);
-    hipLaunchKernelGGL(k_bc_fm<2>, dim3(nblk((long)L.ni * L.nj, 256)), dim3(256), 0, s, L, F, C, tfix, g);
+    const long nfix = lidx_h(L, ifix - 1, jfix - 1, kfix - 1);
+    if (one_sided_copy(C)) {
+        hipLaunchKernelGGL((k_bc_fm<0, 0>), dim3(face_blocks(L, 0, 0)), dim3(256), 0, s, L, F, C, nfix);
+        hipLaunchKernelGGL((k_bc_fm<1, 1>), dim3(face_blocks(L, 1, 1)), dim3(256), 0, s, L, F, C, nfix);
+        hipLaunchKernelGGL((k_bc_fm<2, 2>), dim3(face_blocks(L, 2, 2)), dim3(256), 0, s, L, F, C, nfix);
+    } else {
+        hipLaunchKernelGGL((k_bc_fm<0, 2>), dim3(face_blocks(L, 0, 2)), dim3(256), 0, s, L, F, C, nfix);
+    }
     if (!pfix_deferred) hipLaunchKernelGGL(k_pfix_sub, dim3(nblk(L.n, 256)), dim3(256), 0, s, L, F);
 }
 
@@ -726,8 +826,9 @@ __global__ void k_probe(Fields F, int n, const long* node, double* out) {
 }
 
 void launch_real_residual(hipStream_t s, const Level& L, const Fields& F) {
-    hipLaunchKernelGGL(k_real_part, dim3(kResidBlocks), dim3(256), 0, s, L, F);
-    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(256), 0, s, F, kResidBlocks);
+    const int nb = resid_blocks(L.n);
+    hipLaunchKernelGGL(k_real_part, dim3(nb), dim3(256), 0, s, L, F);
+    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(256), 0, s, F, nb);
 }
 
 void launch_probe(hipStream_t s, const Fields& F, int n, const long* node, double* out) {
@@ -735,8 +836,9 @@ void launch_probe(hipStream_t s, const Fields& F, int n, const long* node, doubl
 }
 
 void launch_resid_and_save(hipStream_t s, const Level& L, const Fields& F, int save, bool pfix) {
-    hipLaunchKernelGGL(k_resid_part, dim3(kResidBlocks), dim3(256), 0, s, L, F, save, pfix ? 1 : 0);
-    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(256), 0, s, F, kResidBlocks);
+    const int nb = resid_blocks(L.n);
+    hipLaunchKernelGGL(k_resid_part, dim3(nb), dim3(256), 0, s, L, F, save, pfix ? 1 : 0);
+    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(256), 0, s, F, nb);
 }
 
 // ---- every zone of a group in one launch per kernel ----
@@ -777,24 +879,31 @@ void launch_prolong_z(hipStream_t s, const ZoneList& Z, int n) {
 
 // bcond_fm faces and the pinned-pressure shift of every zone's fine level
 void launch_bcond_fm_z(hipStream_t s, const ZoneList& Z) {
-    unsigned fi = 0, fj = 0, fk = 0, gn = 0;
-    const ZoneGrid Gi = Z.grid([&](const ZoneDesc& z) { return nblk((long)z.lv[1].nj * z.lv[1].nk, 256); }, fi);
-    const ZoneGrid Gj = Z.grid([&](const ZoneDesc& z) { return nblk((long)z.lv[1].ni * z.lv[1].nk, 256); }, fj);
-    const ZoneGrid Gk = Z.grid([&](const ZoneDesc& z) { return nblk((long)z.lv[1].ni * z.lv[1].nj, 256); }, fk);
+    unsigned gn = 0;
+    bool split = false;
+    for (const ZoneDesc& z : Z.host) split = split || one_sided_copy(z.C);
+    auto faces = [&](auto kernel, int e0, int e1) {
+        unsigned nf = 0;
+        const ZoneGrid G = Z.grid([&](const ZoneDesc& z) { return face_blocks(z.lv[1], e0, e1); }, nf);
+        hipLaunchKernelGGL(kernel, dim3(nf), dim3(256), 0, s, G);
+    };
+    if (split) {
+        faces(k_bc_fm_z<0, 0>, 0, 0);
+        faces(k_bc_fm_z<1, 1>, 1, 1);
+        faces(k_bc_fm_z<2, 2>, 2, 2);
+    } else {
+        faces(k_bc_fm_z<0, 2>, 0, 2);
+    }
     const ZoneGrid Gn = Z.grid([&](const ZoneDesc& z) { return nblk(z.lv[1].n, 256); }, gn);
-    hipLaunchKernelGGL(k_bc_fm_z<0>, dim3(fi), dim3(256), 0, s, Gi);
-    hipLaunchKernelGGL(k_bc_fm_z<1>, dim3(fj), dim3(256), 0, s, Gj);
-    hipLaunchKernelGGL(k_bc_fm_z<2>, dim3(fk), dim3(256), 0, s, Gk);
-    hipLaunchKernelGGL(k_pfix_read_z, dim3(1), dim3(64), 0, s, (const ZoneDesc*)Z.dev, Z.nz());
     hipLaunchKernelGGL(k_pfix_sub_z, dim3(gn), dim3(256), 0, s, Gn);
 }
 
 // update norms of every zone's fine level into its F.resid, then qold <- q
 void launch_resid_and_save_z(hipStream_t s, const ZoneList& Z, int save) {
     unsigned nb = 0;
-    const ZoneGrid G = Z.grid([&](const ZoneDesc&) { return (unsigned)kResidBlocks; }, nb);
+    const ZoneGrid G = Z.grid([&](const ZoneDesc& z) { return (unsigned)resid_blocks(z.lv[1].n); }, nb);
     hipLaunchKernelGGL(k_resid_part_z, dim3(nb), dim3(256), 0, s, G, save);
-    hipLaunchKernelGGL(k_resid_final_z, dim3(Z.nz()), dim3(256), 0, s, (const ZoneDesc*)Z.dev, kResidBlocks);
+    hipLaunchKernelGGL(k_resid_final_z, dim3(Z.nz()), dim3(256), 0, s, (const ZoneDesc*)Z.dev);
 }
 
 void launch_copy_qold(hipStream_t s, const Level& L, const Fields& F) {

@@ -12,7 +12,7 @@
 //   k_sa_sweep<D> the rhs_sa_adi_solver sweeps in i, j and k with every
 //               row on chip (seg_sweep.h); D = 2 also applies the update of
 //               des_eddy.F90:260-272
-//   k_sa_bc<D>  rhs_sa_bcond faces, k_sa_clamp its nu~ floor and xnut
+//   k_sa_bc     rhs_sa_bcond faces, k_sa_clamp its nu~ floor and xnut
 #include <algorithm>
 
 #include "desalm_internal.h"
@@ -25,6 +25,14 @@ namespace {
 // Spalart-Allmaras constants (des_eddy.F90:63-73)
 constexpr double cb1 = 0.1355, cb2 = 0.622, sig = 2.0 / 3.0, capa = 0.41, cw1 = 3.23906782, cw2 = 0.3,
                  cw3h = 64.0, cv1c = 357.911, cv2 = 5.0;
+
+// nu~ as the update between two floors sees it: after the first
+// sub-iteration every node's nu~ counts as raised to the floor of 1e-7
+// (rhs_sa_bcond.F90:279-287).  Storing that took a pass over the level per
+// sub-iteration (14 us on 193x129x129); only the last one is stored (with
+// xnut, which nothing reads in between), and until then whoever reads a nu~
+// of the sub-iteration before raises it (floored).
+__device__ __forceinline__ double nu_floor(double q, bool floored) { return floored ? fmax(1.0e-07, q) : q; }
 
 __device__ __forceinline__ void sa_prep_body(const Level& L, const Fields& F, unsigned bid, unsigned nblk) {
     const long t = (long)xcd_block(bid, nblk) * blockDim.x + threadIdx.x;
@@ -178,8 +186,8 @@ __host__ __device__ inline unsigned sa_gx(const Level& L) { return (unsigned)((L
 __host__ __device__ inline unsigned sa_gy(const Level& L) { return (unsigned)((L.nj - 2 + kQY - 2) / (kQY - 1)); }
 
 // bid: linear workgroup index over (i tile, j tile, k chunk), i fastest
-__device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, const Consts& C, int kc, unsigned bid,
-                                            unsigned nblk) {
+__device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, const Consts& C, int kc, bool floored,
+                                            unsigned bid, unsigned nblk) {
     __shared__ double s_q[3][kQLN];      // nu~ of planes k-1, k, k+1 (slot k mod 3)
     __shared__ double s_m[kQM][kQLN];    // metrics, J of plane k
     __shared__ double s_u[2][kQLN];      // U/J, V/J of plane k
@@ -220,8 +228,8 @@ __device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, con
     // prologue: nu~ of planes kb-1 .. kb+1; metrics, J, U/J, V/J of plane kb
     for (int k = kb - 1; k <= kb + 1; k++) {
         const int sl = k % 3;
-        s_q[sl][own] = own_ok ? ld32(q5, (unsigned)(o + col + sK * k)) : 0.0;
-        if (has_halo) s_q[sl][halo] = halo_ok ? ld32(q5, (unsigned)(o + hc + sK * k)) : 0.0;
+        s_q[sl][own] = own_ok ? nu_floor(ld32(q5, (unsigned)(o + col + sK * k)), floored) : 0.0;
+        if (has_halo) s_q[sl][halo] = halo_ok ? nu_floor(ld32(q5, (unsigned)(o + hc + sK * k)), floored) : 0.0;
     }
     QMet mcur, mh;
     qload_met(F, o + col + sK * kb, own_ok, mcur);
@@ -372,8 +380,8 @@ __device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, con
             if (has_halo) s_u[d][halo] = uh[d];
         }
         if (more) {
-            s_q[slm][own] = qn_o;
-            if (has_halo) s_q[slm][halo] = qn_h;
+            s_q[slm][own] = own_ok ? nu_floor(qn_o, floored) : 0.0;
+            if (has_halo) s_q[slm][halo] = halo_ok ? nu_floor(qn_h, floored) : 0.0;
         }
         mprev = mcur;
         mcur = mnext;
@@ -384,61 +392,92 @@ __device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, con
     }
 }
 
-// rhs_sa_bcond faces (rhs_sa_bcond.F90:40-269); faces of direction D, both sides
-template <int D>
-__device__ __forceinline__ void sa_bc_body(const Level& L, const Fields& F, const Consts& C, unsigned bid) {
-    const int ni = L.ni, nj = L.nj, nk = L.nk;
-    const long sI = 1, sJ = ni, sK = (long)ni * nj;
-    const long t = (long)bid * blockDim.x + threadIdx.x;
-    long nface, base, sD;
-    int nd;
-    if (D == 0) {
-        nface = (long)nj * nk;
-        if (t >= nface) return;
-        base = sJ * (t % nj) + sK * (t / nj);
-        sD = sI;
-        nd = ni;
-    } else if (D == 1) {
-        nface = (long)ni * nk;
-        if (t >= nface) return;
-        base = (t % ni) + sK * (t / ni);
-        sD = sJ;
-        nd = nj;
-    } else {
-        nface = (long)ni * nj;
-        if (t >= nface) return;
-        base = t;
-        sD = sK;
-        nd = nk;
+// rhs_sa_bcond faces (rhs_sa_bcond.F90:40-269): i, then j, then k, in one
+// launch as bcond_fm's are (k_mg.hip): the value of a node after direction E
+// is formed from its sources' values after direction E - 1, and the thread of
+// a node's last direction stores it.  A node that no face writes is read from
+// memory: inside the block this sub-iteration's update, on a boundary plane
+// the value of the one before (floored).
+template <int E>
+struct SaBc {
+    static __device__ __forceinline__ double get(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                 bool floored) {
+        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
+        if (p[E] == 0) return face(L, F, C, p, false, floored);
+        if (p[E] == nd - 1) return face(L, F, C, p, true, floored);
+        return SaBc<E - 1>::get(L, F, C, p, floored);
     }
-    double* q5 = F.q[4] + L.off;
-    const int b0 = 2 * D, b1 = 2 * D + 1;
-    const long lo = base, hi = base + (long)(nd - 1) * sD;
-    switch (C.btype[b0]) {
-        case 1: q5[lo] = 0.0; break;
-        case 2: case 3: q5[lo] = C.sa[b0][0] * q5[lo + sD] + C.sb[b0][0] * q5[lo + 2 * sD]; break;
-        case 6: case 7: q5[lo] = q5[base + (long)(nd - 2) * sD]; break;  // wraps in both
-        case 5: {  // characteristic outlet: extrapolated on the grid ratio (k faces: ratio 0)
-            const double r = D < 2 ? F.rat[b0][t] : 0.0;
-            q5[lo] = (1.0 + r) * q5[lo + sD] - r * q5[lo + 2 * sD];
-            break;
+    static __device__ __forceinline__ double before(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                    int pos, bool floored) {
+        int s[3] = {p[0], p[1], p[2]};
+        s[E] = pos;
+        return SaBc<E - 1>::get(L, F, C, s, floored);
+    }
+    static __device__ __forceinline__ double face(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
+                                                  bool high, bool floored) {
+        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
+        const int bt = high ? C.btype[2 * E + 1] : C.btype[2 * E];
+        const int s1 = high ? nd - 2 : 1, s2 = high ? nd - 3 : 2;
+        switch (bt) {
+            case 1: return 0.0;
+            case 2: case 3: {
+                const double sa = high ? C.sa[2 * E + 1][0] : C.sa[2 * E][0];
+                const double sb = high ? C.sb[2 * E + 1][0] : C.sb[2 * E][0];
+                return sa * before(L, F, C, p, s1, floored) + sb * before(L, F, C, p, s2, floored);
+            }
+            case 6: case 7:  // wraps in both
+                return before(L, F, C, p, high ? 1 : nd - 2, floored);
+            case 8:
+                if (E == 0 && high) return before(L, F, C, p, nd - 2, floored);
+                break;
+            case 5: {  // characteristic outlet: extrapolated on the grid ratio (k faces: ratio 0)
+                const double* rat = high ? F.rat[E < 2 ? 2 * E + 1 : 0] : F.rat[E < 2 ? 2 * E : 0];
+                const double r = E == 0 ? rat[p[1] + (long)L.nj * p[2]] : E == 1 ? rat[p[0] + (long)L.ni * p[2]] : 0.0;
+                return (1.0 + r) * before(L, F, C, p, s1, floored) - r * before(L, F, C, p, s2, floored);
+            }
+            default: break;
         }
-        default: break;
+        return before(L, F, C, p, high ? nd - 1 : 0, floored);
     }
-    switch (C.btype[b1]) {
-        case 1: q5[hi] = 0.0; break;
-        case 2: case 3: q5[hi] = C.sa[b1][0] * q5[hi - sD] + C.sb[b1][0] * q5[hi - 2 * sD]; break;
-        case 6: case 7: q5[hi] = q5[base + sD]; break;
-        case 8:
-            if (D == 0) q5[hi] = q5[hi - sD];
-            break;
-        case 5: {
-            const double r = D < 2 ? F.rat[b1][t] : 0.0;
-            q5[hi] = (1.0 + r) * q5[hi - sD] - r * q5[hi - 2 * sD];
-            break;
-        }
-        default: break;
+};
+template <>
+struct SaBc<-1> {
+    static __device__ __forceinline__ double get(const Level& L, const Fields& F, const Consts&, const int (&p)[3],
+                                                 bool floored) {
+        const bool bnd = p[0] == 0 || p[0] == L.ni - 1 || p[1] == 0 || p[1] == L.nj - 1 || p[2] == 0 || p[2] == L.nk - 1;
+        return nu_floor(F.q[4][L.off + p[0] + (long)L.ni * (p[1] + (long)L.nj * p[2])], floored && bnd);
     }
+};
+template <int E>
+__device__ __forceinline__ void sa_bc_faces(const Level& L, const Fields& F, const Consts& C, long t, bool high,
+                                            bool floored) {
+    const int nd[3] = {L.ni, L.nj, L.nk};
+    const int n0 = E == 0 ? L.nj : L.ni, n1 = E == 2 ? L.nj : L.nk;
+    if (t >= (long)n0 * n1) return;
+    const int a = (int)(t % n0), b = (int)(t / n0);
+    int p[3] = {E == 0 ? 0 : a, E == 0 ? a : E == 1 ? 0 : b, E == 2 ? 0 : b};
+    // nodes on a later direction's face belong to its threads
+    for (int e = E + 1; e < 3; e++)
+        if (p[e] == 0 || p[e] == nd[e] - 1) return;
+    if (high) p[E] = nd[E] - 1;
+    F.q[4][L.off + p[0] + (long)L.ni * (p[1] + (long)L.nj * p[2])] = SaBc<E>::face(L, F, C, p, high, floored);
+}
+__host__ __device__ inline unsigned sa_face_blocks(const Level& L, int e) {
+    const long n = e == 0 ? (long)L.nj * L.nk : e == 1 ? (long)L.ni * L.nk : (long)L.ni * L.nj;
+    return (unsigned)((n + 255) / 256);
+}
+__device__ __forceinline__ void sa_bc_body(const Level& L, const Fields& F, const Consts& C, bool floored,
+                                           unsigned bid) {
+    // even workgroups the low faces, odd ones the high faces
+    const unsigned n0 = sa_face_blocks(L, 0), n1 = sa_face_blocks(L, 1);
+    const bool high = bid & 1u;
+    const unsigned b = bid >> 1;
+    if (b < n0) sa_bc_faces<0>(L, F, C, (long)b * 256 + threadIdx.x, high, floored);
+    else if (b < n0 + n1) sa_bc_faces<1>(L, F, C, (long)(b - n0) * 256 + threadIdx.x, high, floored);
+    else sa_bc_faces<2>(L, F, C, (long)(b - n0 - n1) * 256 + threadIdx.x, high, floored);
+}
+__host__ __device__ inline unsigned sa_bc_blocks(const Level& L) {
+    return 2 * (sa_face_blocks(L, 0) + sa_face_blocks(L, 1) + sa_face_blocks(L, 2));
 }
 
 // nu~ floor and xnut = nu~ fv1 on every node (rhs_sa_bcond.F90:279-291)
@@ -463,7 +502,7 @@ __device__ __forceinline__ void sa_clamp_body(const Level& L, const Fields& F, c
 //   q5 += (-q5 + qold + x) / (1 + 1.5 e_source dtev / delti), qold = q5 here.
 template <int D, int R>
 __device__ __forceinline__ void sa_sweep_body(const Level& L, const Fields& F, const Consts& C, const SegShape& sh,
-                                              unsigned bid) {
+                                              bool floored, unsigned bid) {
     extern __shared__ double smem_sa[];
     const int P = sh.P, TI = sh.TI, n = sh.n;
     const int tid = (int)threadIdx.x;
@@ -565,7 +604,7 @@ __device__ __forceinline__ void sa_sweep_body(const Level& L, const Fields& F, c
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const long g = L.off + base + (long)(min(s0 + r, n - 1) + 1) * sD;
-            qv[r] = F.q[4][g];
+            qv[r] = nu_floor(F.q[4][g], floored);
             dv[r] = F.dtev[g];
         }
 #pragma unroll
@@ -590,30 +629,28 @@ __global__ void __launch_bounds__(256) k_sa_prep_z(ZoneGrid G) {
     sa_prep_body(L, F, b.bid, b.nblk);
 }
 // three waves per SIMD: fits in 168 VGPRs without spilling
-__global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs(Level L, Fields F, Consts C, int kc) {
-    sa_rhs_body(L, F, C, kc, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
+__global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs(Level L, Fields F, Consts C, int kc, int floored) {
+    sa_rhs_body(L, F, C, kc, floored, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
                 gridDim.x * gridDim.y * gridDim.z);
 }
-__global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs_z(ZoneGrid G, int kc) {
+__global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs_z(ZoneGrid G, int kc, int floored) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
     const Level L = Z.lv[1];
     const Fields F = Z.F;
     const Consts C = Z.C;
-    sa_rhs_body(L, F, C, kc, b.bid, b.nblk);
+    sa_rhs_body(L, F, C, kc, floored, b.bid, b.nblk);
 }
-template <int D>
-__global__ void __launch_bounds__(256) k_sa_bc(Level L, Fields F, Consts C) {
-    sa_bc_body<D>(L, F, C, blockIdx.x);
+__global__ void __launch_bounds__(256) k_sa_bc(Level L, Fields F, Consts C, int floored) {
+    sa_bc_body(L, F, C, floored, blockIdx.x);
 }
-template <int D>
-__global__ void __launch_bounds__(256) k_sa_bc_z(ZoneGrid G) {
+__global__ void __launch_bounds__(256) k_sa_bc_z(ZoneGrid G, int floored) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
     const Level L = Z.lv[1];
     const Fields F = Z.F;
     const Consts C = Z.C;
-    sa_bc_body<D>(L, F, C, b.bid);
+    sa_bc_body(L, F, C, floored, b.bid);
 }
 __global__ void __launch_bounds__(256) k_sa_clamp(Level L, Fields F, Consts C) { sa_clamp_body(L, F, C, blockIdx.x); }
 __global__ void __launch_bounds__(256) k_sa_clamp_z(ZoneGrid G) {
@@ -625,17 +662,17 @@ __global__ void __launch_bounds__(256) k_sa_clamp_z(ZoneGrid G) {
     sa_clamp_body(L, F, C, b.bid);
 }
 template <int D, int R>
-__global__ void __launch_bounds__(512) k_sa_sweep(Level L, Fields F, Consts C, SegShape sh) {
-    sa_sweep_body<D, R>(L, F, C, sh, xcd_block(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(512) k_sa_sweep(Level L, Fields F, Consts C, SegShape sh, int floored) {
+    sa_sweep_body<D, R>(L, F, C, sh, floored, xcd_block(blockIdx.x, gridDim.x));
 }
 template <int D, int R>
-__global__ void __launch_bounds__(512) k_sa_sweep_z(ZoneGrid G, int P, int TI) {
+__global__ void __launch_bounds__(512) k_sa_sweep_z(ZoneGrid G, int P, int TI, int floored) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
     const Level L = Z.lv[1];
     const Fields F = Z.F;
     const Consts C = Z.C;
-    sa_sweep_body<D, R>(L, F, C, seg_lines(L, D, P, TI), xcd_block(b.bid, b.nblk));
+    sa_sweep_body<D, R>(L, F, C, seg_lines(L, D, P, TI), floored, xcd_block(b.bid, b.nblk));
 }
 
 }  // namespace
@@ -649,16 +686,16 @@ void launch_sa_prep(hipStream_t s, const Level& L, const Fields& F) {
     hipLaunchKernelGGL(k_sa_prep, dim3((unsigned)((L.n + b - 1) / b)), dim3(b), 0, s, L, F);
 }
 
-void launch_sa_rhs(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int kc) {
+void launch_sa_rhs(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int kc, bool floored) {
     if (kc <= 0) kc = sa_kc_default(L);
     kc = std::min(kc, L.nk - 2);
     const dim3 gq(sa_gx(L), sa_gy(L), (unsigned)((L.nk - 2 + kc - 1) / kc));
-    hipLaunchKernelGGL(k_sa_rhs, gq, dim3(kQX * kQY), 0, s, L, F, C, kc);
+    hipLaunchKernelGGL(k_sa_rhs, gq, dim3(kQX * kQY), 0, s, L, F, C, kc, (int)floored);
 }
 
 // the ADI sweep of direction D over the interior lines of the fine level
 template <int D>
-static void sa_sweep(hipStream_t s, const Level& L, const Fields& F, const Consts& C) {
+static void sa_sweep(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int floored) {
     const int n = D == 0 ? L.ni - 2 : D == 1 ? L.nj - 2 : L.nk - 2;
     const long nl = D == 0 ? (long)(L.nj - 2) * (L.nk - 2) : D == 1 ? (long)(L.ni - 2) * (L.nk - 2)
                                                                     : (long)(L.ni - 2) * (L.nj - 2);
@@ -671,34 +708,31 @@ static void sa_sweep(hipStream_t s, const Level& L, const Fields& F, const Const
     const unsigned nb = (unsigned)((sh.nlines + sh.TI - 1) / sh.TI);
     const size_t lds = seg_lds_bytes(sh, 1);
     if (R == 4)
-        hipLaunchKernelGGL((k_sa_sweep<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, C, sh);
+        hipLaunchKernelGGL((k_sa_sweep<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, C, sh, floored);
     else
-        hipLaunchKernelGGL((k_sa_sweep<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, C, sh);
+        hipLaunchKernelGGL((k_sa_sweep<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, C, sh, floored);
 }
 
 void launch_des_eddy(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int itk, int kc) {
     const int b = 256;
     const unsigned gn = (unsigned)((L.n + b - 1) / b);
     launch_sa_prep(s, L, F);
-    const unsigned fi = (unsigned)(((long)L.nj * L.nk + b - 1) / b);
-    const unsigned fj = (unsigned)(((long)L.ni * L.nk + b - 1) / b);
-    const unsigned fk = (unsigned)(((long)L.ni * L.nj + b - 1) / b);
+    const unsigned nf = sa_bc_blocks(L);
     for (int it = 0; it < itk; it++) {
-        launch_sa_rhs(s, L, F, C, kc);
-        sa_sweep<0>(s, L, F, C);
-        sa_sweep<1>(s, L, F, C);
-        sa_sweep<2>(s, L, F, C);
-        hipLaunchKernelGGL(k_sa_bc<0>, dim3(fi), dim3(b), 0, s, L, F, C);
-        hipLaunchKernelGGL(k_sa_bc<1>, dim3(fj), dim3(b), 0, s, L, F, C);
-        hipLaunchKernelGGL(k_sa_bc<2>, dim3(fk), dim3(b), 0, s, L, F, C);
-        hipLaunchKernelGGL(k_sa_clamp, dim3(gn), dim3(b), 0, s, L, F, C);
+        const int floored = it > 0;
+        launch_sa_rhs(s, L, F, C, kc, floored);
+        sa_sweep<0>(s, L, F, C, floored);
+        sa_sweep<1>(s, L, F, C, floored);
+        sa_sweep<2>(s, L, F, C, floored);
+        hipLaunchKernelGGL(k_sa_bc, dim3(nf), dim3(b), 0, s, L, F, C, floored);
     }
+    if (itk > 0) hipLaunchKernelGGL(k_sa_clamp, dim3(gn), dim3(b), 0, s, L, F, C);
 }
 
 // the ADI sweep of direction D over every zone of a group in one launch,
 // with the segment count of the longest line
 template <int D>
-static void sa_sweep_z(hipStream_t s, const ZoneList& Z) {
+static void sa_sweep_z(hipStream_t s, const ZoneList& Z, int floored) {
     int len = 0;
     for (const ZoneDesc& z : Z.host) len = std::max(len, seg_lines(z.lv[1], D, 1, 1).n);
     const int R = len <= 64 ? 4 : 8;
@@ -709,20 +743,18 @@ static void sa_sweep_z(hipStream_t s, const ZoneList& Z) {
         nb);
     const size_t lds = seg_lds_bytes(sh, 1);
     if (R == 4)
-        hipLaunchKernelGGL((k_sa_sweep_z<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, G, sh.P, sh.TI);
+        hipLaunchKernelGGL((k_sa_sweep_z<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, G, sh.P, sh.TI, floored);
     else
-        hipLaunchKernelGGL((k_sa_sweep_z<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, G, sh.P, sh.TI);
+        hipLaunchKernelGGL((k_sa_sweep_z<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, G, sh.P, sh.TI, floored);
 }
 
 // des_eddy on the fine level of every zone of a group, one launch per kernel
 void launch_des_eddy_z(hipStream_t s, const ZoneList& Z, int itk, int kc) {
     const int b = 256;
     auto nodes = [&](const ZoneDesc& z) { return (unsigned)((z.lv[1].n + b - 1) / b); };
-    unsigned gn = 0, fi = 0, fj = 0, fk = 0, gq = 0;
+    unsigned gn = 0, nf = 0, gq = 0;
     const ZoneGrid Gn = Z.grid(nodes, gn);
-    const ZoneGrid Gi = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].nj * z.lv[1].nk + b - 1) / b); }, fi);
-    const ZoneGrid Gj = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].ni * z.lv[1].nk + b - 1) / b); }, fj);
-    const ZoneGrid Gk = Z.grid([&](const ZoneDesc& z) { return (unsigned)(((long)z.lv[1].ni * z.lv[1].nj + b - 1) / b); }, fk);
+    const ZoneGrid Gf = Z.grid([&](const ZoneDesc& z) { return sa_bc_blocks(z.lv[1]); }, nf);
     // one plane count from the tiles of all zones (as k_visc_pk's: 502 us at
     // the one plane of the smallest of six blocks' own default, 400 us at nine)
     if (kc <= 0) {
@@ -736,15 +768,14 @@ void launch_des_eddy_z(hipStream_t s, const ZoneList& Z, int itk, int kc) {
         gq);
     hipLaunchKernelGGL(k_sa_prep_z, dim3(gn), dim3(b), 0, s, Gn);
     for (int it = 0; it < itk; it++) {
-        hipLaunchKernelGGL(k_sa_rhs_z, dim3(gq), dim3(kQX * kQY), 0, s, Gq, kc);
-        sa_sweep_z<0>(s, Z);
-        sa_sweep_z<1>(s, Z);
-        sa_sweep_z<2>(s, Z);
-        hipLaunchKernelGGL(k_sa_bc_z<0>, dim3(fi), dim3(b), 0, s, Gi);
-        hipLaunchKernelGGL(k_sa_bc_z<1>, dim3(fj), dim3(b), 0, s, Gj);
-        hipLaunchKernelGGL(k_sa_bc_z<2>, dim3(fk), dim3(b), 0, s, Gk);
-        hipLaunchKernelGGL(k_sa_clamp_z, dim3(gn), dim3(b), 0, s, Gn);
+        const int floored = it > 0;
+        hipLaunchKernelGGL(k_sa_rhs_z, dim3(gq), dim3(kQX * kQY), 0, s, Gq, kc, floored);
+        sa_sweep_z<0>(s, Z, floored);
+        sa_sweep_z<1>(s, Z, floored);
+        sa_sweep_z<2>(s, Z, floored);
+        hipLaunchKernelGGL(k_sa_bc_z, dim3(nf), dim3(b), 0, s, Gf, floored);
     }
+    if (itk > 0) hipLaunchKernelGGL(k_sa_clamp_z, dim3(gn), dim3(b), 0, s, Gn);
 }
 
 }  // namespace desalm

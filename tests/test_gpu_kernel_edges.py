@@ -86,3 +86,29 @@ def test_line_sweep_segments(gpu, dims, prec):
     assert po.relerr(x, xo) <= tol
     assert s.pivot_events == 0
     s.close()
+
+
+@pytest.mark.parametrize("itk", [1, 3])
+@pytest.mark.parametrize("bt", [(1, 8, 6, 1, 3, 2), (4, 8, 1, 6, 6, 2), (3, 2, 4, 0, 4, 4), (0, 1, 6, 6, 1, 6),
+                                (5, 3, 5, 4, 5, 0), (2, 0, 0, 3, 6, 6), (7, 7, 1, 4, 7, 7)])
+def test_boundary_faces_in_one_launch(gpu, bt, itk):
+    """Edge and corner nodes take the i, then j, then k rules in one launch:
+    mixed types on adjacent faces, plane copies on one face only (their own
+    launches), pinned node on a corner, nu~ below its floor at the start, one
+    and three SA sub-iterations (the floor is stored by the last)."""
+    c = cases.wavy(11, 9, 13, ng=2, itm=2, des=True, itk=itk, btype=bt, amp=0.02, iters=(1, 2))
+    c.params.ifix, c.params.jfix, c.params.kfix = 1, 9, 1
+    c.q[::7, 4] = 1e-9
+    s = Solver(c.params).load_case(c)
+    s.mg_driver()
+    q, _, _, x = s.get_state()
+    o = po.Oracle(c.params).load_case(c)
+    o.mg_driver()
+    qo, _, _, xo = o.get_state()
+    assert max(po.relerr(q[:, m], qo[:, m]) for m in range(5)) <= 1e-10
+    assert po.relerr(x, xo) <= 1e-10
+    # the coarsest level's residual, formed once after the last pseudo-iteration
+    rh = s.level_field("rh", 2)
+    off = o.level_offset(2)
+    assert po.relerr(rh, o.get("rh")[off:off + len(rh)]) <= 1e-10
+    s.close()
