@@ -359,64 +359,56 @@ __global__ void k_outlet_ratio(Level L, Fields F, int b, int dir) {
 // Inflow (btype 4) on a k face uses ratio 0: the reference fills its table
 // only where btype == 4 .and. btype == 5 (init.F90:2855, :2874), i.e. never,
 // and the table is zero as allocated.
+// (The rule of a face is first reduced to at most three source positions, so
+// that one level of the recursion has three call sites and not one per rule.)
 template <int E0, int E>
 struct BcValue {
     // q(1:4) after directions E0 .. E at node p
     static __device__ __forceinline__ void get(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
                                                double (&v)[4]) {
         const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
-        if (p[E] == 0) low(L, F, C, p, v);
-        else if (p[E] == nd - 1) high(L, F, C, p, v);
-        else BcValue<E0, E - 1>::get(L, F, C, p, v);
-    }
-    static __device__ __forceinline__ void before(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                                  int pos, double (&v)[4]) {
+        // the rule at p: a copy of s0, or a combination of s1 and s2 (all of q,
+        // or the pressure alone with the rest as in a copy)
+        bool high = p[E] == nd - 1;
+        const bool face = p[E] == 0 || high;
+        int bt = face ? (high ? C.btype[2 * E + 1] : C.btype[2 * E]) : 0;
+        if (E > 0 && high && bt == 6) {  // the low plane as it is by now
+            high = false;
+            bt = C.btype[2 * E];
+        }
+        int s0 = face ? (high ? nd - 1 : 0) : p[E];
+        if (bt == 6 && E > 0) s0 = nd - 1;  // plane copy from the opposite boundary plane (not done for i)
+        if (bt == 7) s0 = high ? 1 : nd - 2;  // periodic wrap: the image of the opposite interior plane
+        if (bt == 8 && E == 0 && high) s0 = nd - 2;
+        const bool lin = bt >= 1 && bt <= 3, inflow = bt == 4;
         int s[3] = {p[0], p[1], p[2]};
-        s[E] = pos;
-        BcValue<E0, E - 1>::get(L, F, C, s, v);
-    }
-    // grid ratio of an inflow face at node p
-    static __device__ __forceinline__ double ratio(const Level& L, const Fields& F, int b, const int (&p)[3]) {
-        if (E == 2) return 0.0;
-        return E == 0 ? F.rat[b][p[1] + (long)L.nj * p[2]] : F.rat[b][p[0] + (long)L.ni * p[2]];
-    }
-    // the common rules of face b, node pos on it, s one node off it, s2 two
-    static __device__ __forceinline__ void face(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                                int bt, int b, int pos, int s, int s2, double (&v)[4]) {
-        double a[4], c[4];
-        if (bt >= 1 && bt <= 3) {
-            before(L, F, C, p, s, a);
-            before(L, F, C, p, s2, c);
+        double a[4] = {}, c[4] = {};
+        if (!lin) {
+            s[E] = s0;
+            BcValue<E0, E - 1>::get(L, F, C, s, v);
+        }
+        if (lin || inflow) {
+            s[E] = high ? nd - 2 : 1;
+            BcValue<E0, E - 1>::get(L, F, C, s, a);
+            s[E] = high ? nd - 3 : 2;
+            BcValue<E0, E - 1>::get(L, F, C, s, c);
+        }
+        if (lin) {
 #pragma unroll
-            for (int m = 0; m < 4; m++) v[m] = C.sa[b][m] * a[m] + C.sb[b][m] * c[m];
-        } else {
-            before(L, F, C, p, pos, v);
-            if (bt == 4) {  // inflow: pressure extrapolated on the grid ratio (bcond_fm.F90:95-102)
-                const double r = ratio(L, F, b, p);
-                before(L, F, C, p, s, a);
-                before(L, F, C, p, s2, c);
-                v[0] = (1.0 + r) * a[0] - r * c[0];
+            for (int m = 0; m < 4; m++) {
+                const double sa = high ? C.sa[2 * E + 1][m] : C.sa[2 * E][m];
+                const double sb = high ? C.sb[2 * E + 1][m] : C.sb[2 * E][m];
+                v[m] = fma(sa, a[m], sb * c[m]);
             }
         }
-    }
-    static __device__ __forceinline__ void low(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                               double (&v)[4]) {
-        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
-        const int bt = C.btype[2 * E];
-        // plane copy from the opposite boundary plane (not done for i);
-        // periodic wrap: the image of the opposite interior plane
-        if (bt == 6 && E > 0) before(L, F, C, p, nd - 1, v);
-        else if (bt == 7) before(L, F, C, p, nd - 2, v);
-        else face(L, F, C, p, bt, 2 * E, 0, 1, 2, v);
-    }
-    static __device__ __forceinline__ void high(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                                double (&v)[4]) {
-        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
-        const int bt = C.btype[2 * E + 1];
-        if (bt == 6 && E > 0) low(L, F, C, p, v);  // the low plane as it is by now
-        else if (bt == 7) before(L, F, C, p, 1, v);
-        else if (bt == 8 && E == 0) before(L, F, C, p, nd - 2, v);
-        else face(L, F, C, p, bt, 2 * E + 1, nd - 1, nd - 2, nd - 3, v);
+        if (inflow) {  // pressure extrapolated on the grid ratio (bcond_fm.F90:95-102)
+            double r = 0.0;
+            if (E < 2) {
+                const double* rat = high ? F.rat[E < 2 ? 2 * E + 1 : 0] : F.rat[E < 2 ? 2 * E : 0];
+                r = E == 0 ? rat[p[1] + (long)L.nj * p[2]] : rat[p[0] + (long)L.ni * p[2]];
+            }
+            v[0] = fma(1.0 + r, a[0], -(r * c[0]));
+        }
     }
 };
 // before the first direction: memory
@@ -468,7 +460,7 @@ __device__ __forceinline__ void bc_store(const Level& L, const Fields& F, const 
     // nodes on a later direction's face belong to its threads
     for (int e = E + 1; e <= E1; e++)
         if (p[e] == 0 || p[e] == nd[e] - 1) return;
-    double a[4], b[4];
+    double a[4];
     if (side != 2) {
         if (side) p[E] = nd[E] - 1;
         BcValue<E0, E>::get(L, F, C, p, a);
@@ -477,10 +469,11 @@ __device__ __forceinline__ void bc_store(const Level& L, const Fields& F, const 
         for (int m = 0; m < 4; m++) F.q[m][g] = a[m];
         return;
     }
-    BcValue<E0, E>::low(L, F, C, p, a);
+    double b[4];
+    BcValue<E0, E>::get(L, F, C, p, a);
     const long lo = L.off + lidx(L, p[0], p[1], p[2]);
     p[E] = nd[E] - 1;
-    BcValue<E0, E>::high(L, F, C, p, b);
+    BcValue<E0, E>::get(L, F, C, p, b);
     const long hi = L.off + lidx(L, p[0], p[1], p[2]);
     // one launch per direction: the pinned node's pressure comes from the
     // thread of its k line, since a one-sided plane copy to it reads the plane

@@ -403,41 +403,29 @@ struct SaBc {
     static __device__ __forceinline__ double get(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
                                                  bool floored) {
         const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
-        if (p[E] == 0) return face(L, F, C, p, false, floored);
-        if (p[E] == nd - 1) return face(L, F, C, p, true, floored);
-        return SaBc<E - 1>::get(L, F, C, p, floored);
-    }
-    static __device__ __forceinline__ double before(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                                    int pos, bool floored) {
+        const bool high = p[E] == nd - 1;
+        const bool face = p[E] == 0 || high;
+        const int bt = face ? (high ? C.btype[2 * E + 1] : C.btype[2 * E]) : 0;
+        if (bt == 1) return 0.0;
+        // a copy of s0, or a combination of the two nodes off the face
         int s[3] = {p[0], p[1], p[2]};
-        s[E] = pos;
-        return SaBc<E - 1>::get(L, F, C, s, floored);
-    }
-    static __device__ __forceinline__ double face(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
-                                                  bool high, bool floored) {
-        const int nd = E == 0 ? L.ni : E == 1 ? L.nj : L.nk;
-        const int bt = high ? C.btype[2 * E + 1] : C.btype[2 * E];
-        const int s1 = high ? nd - 2 : 1, s2 = high ? nd - 3 : 2;
-        switch (bt) {
-            case 1: return 0.0;
-            case 2: case 3: {
-                const double sa = high ? C.sa[2 * E + 1][0] : C.sa[2 * E][0];
-                const double sb = high ? C.sb[2 * E + 1][0] : C.sb[2 * E][0];
-                return sa * before(L, F, C, p, s1, floored) + sb * before(L, F, C, p, s2, floored);
-            }
-            case 6: case 7:  // wraps in both
-                return before(L, F, C, p, high ? 1 : nd - 2, floored);
-            case 8:
-                if (E == 0 && high) return before(L, F, C, p, nd - 2, floored);
-                break;
-            case 5: {  // characteristic outlet: extrapolated on the grid ratio (k faces: ratio 0)
+        if (bt == 2 || bt == 3 || bt == 5) {
+            s[E] = high ? nd - 2 : 1;
+            const double a = SaBc<E - 1>::get(L, F, C, s, floored);
+            s[E] = high ? nd - 3 : 2;
+            const double c = SaBc<E - 1>::get(L, F, C, s, floored);
+            if (bt == 5) {  // characteristic outlet: extrapolated on the grid ratio (k faces: ratio 0)
                 const double* rat = high ? F.rat[E < 2 ? 2 * E + 1 : 0] : F.rat[E < 2 ? 2 * E : 0];
                 const double r = E == 0 ? rat[p[1] + (long)L.nj * p[2]] : E == 1 ? rat[p[0] + (long)L.ni * p[2]] : 0.0;
-                return (1.0 + r) * before(L, F, C, p, s1, floored) - r * before(L, F, C, p, s2, floored);
+                return (1.0 + r) * a - r * c;
             }
-            default: break;
+            const double sa = high ? C.sa[2 * E + 1][0] : C.sa[2 * E][0];
+            const double sb = high ? C.sb[2 * E + 1][0] : C.sb[2 * E][0];
+            return sa * a + sb * c;
         }
-        return before(L, F, C, p, high ? nd - 1 : 0, floored);
+        if (bt == 6 || bt == 7) s[E] = high ? 1 : nd - 2;  // wraps in both
+        if (bt == 8 && E == 0 && high) s[E] = nd - 2;
+        return SaBc<E - 1>::get(L, F, C, s, floored);
     }
 };
 template <>
@@ -460,7 +448,7 @@ __device__ __forceinline__ void sa_bc_faces(const Level& L, const Fields& F, con
     for (int e = E + 1; e < 3; e++)
         if (p[e] == 0 || p[e] == nd[e] - 1) return;
     if (high) p[E] = nd[E] - 1;
-    F.q[4][L.off + p[0] + (long)L.ni * (p[1] + (long)L.nj * p[2])] = SaBc<E>::face(L, F, C, p, high, floored);
+    F.q[4][L.off + p[0] + (long)L.ni * (p[1] + (long)L.nj * p[2])] = SaBc<E>::get(L, F, C, p, floored);
 }
 __host__ __device__ inline unsigned sa_face_blocks(const Level& L, int e) {
     const long n = e == 0 ? (long)L.nj * L.nk : e == 1 ? (long)L.ni * L.nk : (long)L.ni * L.nj;
