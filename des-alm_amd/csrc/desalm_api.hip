@@ -332,8 +332,7 @@ int copy_out_level(desalm_ctx* c, double* const* soa, int ncomp, double* host, c
     for (int m = 0; m < ncomp; m++) src[m] = soa[m] + L.off;
     launch_soa_to_aos(c->stream, src, ncomp, L.n, c->staging);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(host, c->staging, sizeof(double) * ncomp * L.n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, host_read(host, c->staging, sizeof(double) * ncomp * L.n, c->stream, c->device));
     return 0;
 }
 
@@ -357,8 +356,9 @@ int desalm_init(const desalm_params* p, int device, desalm_ctx** out) {
     c->p = *p;
     c->device = device;
     c->ng = p->ng;
-    if (hipSetDevice(device) != hipSuccess) { delete c; return fail(nullptr, "hipSetDevice failed"); }
-    if (hipStreamCreate(&c->stream) != hipSuccess) { delete c; return fail(nullptr, "hipStreamCreate failed"); }
+    host_read_users(1);
+    if (hipSetDevice(device) != hipSuccess) { host_read_users(-1); delete c; return fail(nullptr, "hipSetDevice failed"); }
+    if (hipStreamCreate(&c->stream) != hipSuccess) { host_read_users(-1); delete c; return fail(nullptr, "hipStreamCreate failed"); }
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         desalm_finalize(c);
         return fail(nullptr, "hipEventCreate failed");
@@ -578,10 +578,7 @@ int desalm_get_state(desalm_ctx* c, double* q, double* qn, double* qnm1, double*
     if (copy_out_level(c, c->F.q, 5, q, L)) return -1;
     if (copy_out_level(c, c->F.qn, 5, qn, L)) return -1;
     if (copy_out_level(c, c->F.qnm1, 5, qnm1, L)) return -1;
-    if (xnut) {
-        HIPCHK(c, hipMemcpyAsync(xnut, c->F.xnut, sizeof(double) * c->n1, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-    }
+    if (xnut) HIPCHK(c, host_read(xnut, c->F.xnut, sizeof(double) * c->n1, c->stream, c->device));
     return 0;
 }
 
@@ -1068,33 +1065,30 @@ int desalm_gtsv_batch(int n, int nsys, double* dl, double* d, double* du, double
     if (n < 0 || nsys < 0) return fail(nullptr, "negative size");
     if (n == 0 || nsys == 0) return 0;
     if (!dl || !d || !du || !b) return fail(nullptr, "null argument");
-    const size_t bytes = sizeof(double) * (size_t)n * nsys;
-    double *ddl = nullptr, *dd = nullptr, *ddu = nullptr, *db = nullptr;
-    int* dinfo = nullptr;
-    int rc = 0;
-    if (hipMalloc(&ddl, bytes) != hipSuccess || hipMalloc(&dd, bytes) != hipSuccess ||
-        hipMalloc(&ddu, bytes) != hipSuccess || hipMalloc(&db, bytes) != hipSuccess ||
-        hipMalloc(&dinfo, sizeof(int) * nsys) != hipSuccess) {
-        rc = fail(nullptr, "device allocation failed");
-    } else if (hipMemcpy(ddl, dl, bytes, hipMemcpyHostToDevice) != hipSuccess ||
-               hipMemcpy(dd, d, bytes, hipMemcpyHostToDevice) != hipSuccess ||
-               hipMemcpy(ddu, du, bytes, hipMemcpyHostToDevice) != hipSuccess ||
-               hipMemcpy(db, b, bytes, hipMemcpyHostToDevice) != hipSuccess) {
+    // one allocation: the four arrays, then INFO
+    const size_t len = (size_t)n * nsys, bytes = sizeof(double) * len;
+    double* buf = nullptr;
+    int rc = 0, dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipMalloc(&buf, 4 * bytes + sizeof(int) * nsys) != hipSuccess)
+        return fail(nullptr, "device allocation failed");
+    double* const h[4] = {dl, d, du, b};
+    int* dinfo = (int*)(buf + 4 * len);
+    bool ok = true;
+    for (int k = 0; k < 4 && ok; k++) ok = hipMemcpy(buf + k * len, h[k], bytes, hipMemcpyHostToDevice) == hipSuccess;
+    if (!ok) {
         rc = fail(nullptr, "gtsv: host-to-device copy failed");
     } else {
-        launch_gtsv_batch(0, n, nsys, ddl, dd, ddu, db, dinfo);
+        launch_gtsv_batch(0, n, nsys, buf, buf + len, buf + 2 * len, buf + 3 * len, dinfo);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
             rc = fail(nullptr, "gtsv kernel failed");
-        } else if (hipMemcpy(dl, ddl, bytes, hipMemcpyDeviceToHost) != hipSuccess ||
-                   hipMemcpy(d, dd, bytes, hipMemcpyDeviceToHost) != hipSuccess ||
-                   hipMemcpy(du, ddu, bytes, hipMemcpyDeviceToHost) != hipSuccess ||
-                   hipMemcpy(b, db, bytes, hipMemcpyDeviceToHost) != hipSuccess ||
-                   (info_out && hipMemcpy(info_out, dinfo, sizeof(int) * nsys, hipMemcpyDeviceToHost) != hipSuccess)) {
-            rc = fail(nullptr, "gtsv: device-to-host copy failed");
+        } else {
+            for (int k = 0; k < 4 && ok; k++) ok = host_read(h[k], buf + k * len, bytes, 0, dev) == hipSuccess;
+            if (!ok || (info_out && hipMemcpy(info_out, dinfo, sizeof(int) * nsys, hipMemcpyDeviceToHost) != hipSuccess))
+                rc = fail(nullptr, "gtsv: device-to-host copy failed");
         }
     }
     // teardown: a failing free leaves nothing to recover
-    (void)hipFree(ddl); (void)hipFree(dd); (void)hipFree(ddu); (void)hipFree(db); (void)hipFree(dinfo);
+    (void)hipFree(buf);
     return rc;
 }
 
@@ -2045,6 +2039,7 @@ int desalm_finalize(desalm_ctx* c) {
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    host_read_users(-1);
     return 0;
 }
 

@@ -112,3 +112,31 @@ def test_boundary_faces_in_one_launch(gpu, bt, itk):
     off = o.level_offset(2)
     assert po.relerr(rh, o.get("rh")[off:off + len(rh)]) <= 1e-10
     s.close()
+
+
+@pytest.mark.parametrize("dims", [(47, 47, 47), (48, 47, 47), (53, 53, 56), (53, 53, 57), (101, 67, 67)])
+def test_state_comes_back_through_the_ring(gpu, dims):
+    """Read-backs below and above the 4 MiB of a plain copy, one chunk above
+    a whole number of 2 MiB chunks and longer than the pinned ring: the state
+    that went in comes back, from two threads at once too."""
+    import threading
+    n = dims[0] * dims[1] * dims[2]
+    rng = np.random.default_rng(n)
+    c = cases.wavy(*dims, ng=1, itm=1)
+    sv = [Solver(c.params) for _ in range(2)]
+    st = [[rng.standard_normal((n, 5)) for _ in range(3)] + [rng.standard_normal(n)] for _ in sv]
+    for s, a in zip(sv, st):
+        s.set_state(*a)
+    got = [None, None]
+
+    def read(k):
+        got[k] = sv[k].get_state()
+
+    t = [threading.Thread(target=read, args=(k,)) for k in range(2)]
+    [x.start() for x in t]
+    [x.join() for x in t]
+    for a, g in zip(st, got):
+        assert all(np.array_equal(u, v) for u, v in zip(a, g))
+    for s, a in zip(sv, st):
+        assert np.array_equal(s.level_field("q"), a[0])
+        s.close()
