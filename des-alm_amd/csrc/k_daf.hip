@@ -855,68 +855,157 @@ __global__ void __launch_bounds__(512) k_daf_sweep_z(ZoneGrid G, int n, int P, i
 }
 
 // ---- batched LAPACK SGTSV (src/sgtsv.f:89-259) in FP64, one system per thread ----
-__global__ void k_gtsv_batch(int n, int nsys, double* dl, double* d, double* du, double* b, int* info) {
-    const int sidx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sidx >= nsys) return;
-    double* DL = dl + (long)sidx * n;
-    double* D = d + (long)sidx * n;
-    double* DU = du + (long)sidx * n;
-    double* B = b + (long)sidx * n;
-    int inf = 0;
-    for (int i = 0; i < n - 2 && !inf; i++) {
-        if (fabs(D[i]) >= fabs(DL[i])) {
-            if (D[i] != 0.0) {
-                const double fact = DL[i] / D[i];
-                D[i + 1] = D[i + 1] - fact * DU[i];
-                B[i + 1] = B[i + 1] - fact * B[i];
-            } else {
-                inf = i + 1;
-                break;
-            }
-            DL[i] = 0.0;
-        } else {
-            const double fact = D[i] / DL[i];
-            D[i] = DL[i];
-            double temp = D[i + 1];
-            D[i + 1] = DU[i] - fact * temp;
-            DL[i] = DU[i + 1];
-            DU[i + 1] = -fact * DL[i];
-            DU[i] = temp;
-            temp = B[i];
-            B[i] = B[i + 1];
-            B[i + 1] = temp - fact * B[i + 1];
-        }
-    }
-    if (!inf && n > 1) {
-        const int i = n - 2;
-        if (fabs(D[i]) >= fabs(DL[i])) {
-            if (D[i] != 0.0) {
-                const double fact = DL[i] / D[i];
-                D[i + 1] = D[i + 1] - fact * DU[i];
-                B[i + 1] = B[i + 1] - fact * B[i];
-            } else {
-                inf = i + 1;
-            }
-        } else {
-            const double fact = D[i] / DL[i];
-            D[i] = DL[i];
-            const double temp = D[i + 1];
-            D[i + 1] = DU[i] - fact * temp;
-            DU[i] = temp;
-            const double tb = B[i];
-            B[i] = B[i + 1];
-            B[i + 1] = tb - fact * B[i + 1];
-        }
-    }
-    if (!inf && n > 0 && D[n - 1] == 0.0) inf = n;
-    if (!inf && n > 0) {
-        B[n - 1] = B[n - 1] / D[n - 1];
-        if (n > 1) B[n - 2] = (B[n - 2] - DU[n - 2] * B[n - 1]) / D[n - 2];
-        for (int i = n - 3; i >= 0; i--) B[i] = (B[i] - DU[i] * B[i + 1] - DL[i] * B[i + 2]) / D[i];
-    }
-    if (info) info[sidx] = inf;
-}
+//
+// A system's rows are consecutive in memory, so the threads of a wave, one
+// system each, are n rows apart: read straight from memory every row cost a
+// latency of its own and every access a cache line per thread (2048 systems of
+// 127 rows: 256 us; 16129 of 191: 485 us).  A wave of 64 systems instead moves
+// chunks of kGtRows rows through LDS, in runs of 128 bytes per system, loads
+// the next chunk while it eliminates the current one, and keeps the row that
+// the next row's elimination changes in registers.  Bound by the serial chain
+// of the recurrence (a division and two multiply-adds per row and direction):
+// 2048 systems of 127 rows 83 us, 16129 of 191 131 us.
+constexpr int kGtRows = 16, kGtLd = kGtRows + 1;
 
+__global__ void __launch_bounds__(64) k_gtsv_batch(int n, int nsys, double* dl, double* d, double* du, double* b,
+                                                   int* info) {
+    __shared__ double lds[4][64][kGtLd];
+    const int lane = (int)threadIdx.x;
+    const long s0 = (long)blockIdx.x * 64;
+    const bool act = s0 + lane < nsys;
+    const int ls = lane / kGtRows, lr = lane % kGtRows;  // system and row of this lane's loads and stores
+    constexpr int NQ = kGtRows;
+    double* const arr[4] = {dl, d, du, b};
+    // rows c0 .. of every system of the wave; past the end the last row or
+    // system again
+    double v[4][NQ];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const long sys = min(s0 + ls + 64 / kGtRows * q, (long)nsys - 1);
+            const long g = sys * n + max(0, min(c0 + lr, n - 1));
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k][q] = arr[k][g];
+        }
+    };
+    auto to_lds = [&] {
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) lds[k][ls + 64 / kGtRows * q][lr] = v[k][q];
+    };
+    // forward elimination: row r - 1 is finished by row r
+    int inf = 0;
+    double L0 = 0.0, D0 = 0.0, U0 = 0.0, B0 = 0.0;  // row r - 1
+    load(0);
+    for (int c0 = 0; c0 < n; c0 += kGtRows) {
+        to_lds();
+        __syncthreads();
+        load(c0 + kGtRows);
+        const int nr = min(kGtRows, n - c0);
+        for (int r = 0; r < nr; r++) {
+            const int row = c0 + r;
+            const double L1 = lds[0][lane][r];
+            double D1 = lds[1][lane][r], U1 = lds[2][lane][r], B1 = lds[3][lane][r];
+            if (row > 0) {
+                const bool last = row == n - 1;  // the last elimination has no DU of its second row
+                if (!inf) {
+                    if (fabs(D0) >= fabs(L0)) {
+                        if (D0 != 0.0) {
+                            const double fact = L0 / D0;
+                            D1 = D1 - fact * U0;
+                            B1 = B1 - fact * B0;
+                            if (!last) L0 = 0.0;
+                        } else {
+                            inf = row;
+                        }
+                    } else {
+                        const double fact = D0 / L0;
+                        D0 = L0;
+                        const double td = D1, tb = B0;
+                        D1 = U0 - fact * td;
+                        if (!last) {
+                            L0 = U1;
+                            U1 = -fact * L0;
+                        }
+                        U0 = td;
+                        B0 = B1;
+                        B1 = tb - fact * B1;
+                    }
+                }
+                if (r > 0) {
+                    lds[0][lane][r - 1] = L0;
+                    lds[1][lane][r - 1] = D0;
+                    lds[2][lane][r - 1] = U0;
+                    lds[3][lane][r - 1] = B0;
+                } else if (act) {  // the chunk before is stored already, without its last row
+                    const long g = (s0 + lane) * n + row - 1;
+                    dl[g] = L0;
+                    d[g] = D0;
+                    du[g] = U0;
+                    b[g] = B0;
+                }
+            }
+            L0 = L1;
+            D0 = D1;
+            U0 = U1;
+            B0 = B1;
+        }
+        const bool end = c0 + nr == n;
+        if (end) {
+            lds[0][lane][nr - 1] = L0;
+            lds[1][lane][nr - 1] = D0;
+            lds[2][lane][nr - 1] = U0;
+            lds[3][lane][nr - 1] = B0;
+        }
+        __syncthreads();
+        if (lr < (end ? nr : nr - 1)) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                const int sys = ls + 64 / kGtRows * q;
+                if (s0 + sys < nsys) {
+                    const long g = (s0 + sys) * n + c0 + lr;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) arr[k][g] = lds[k][sys][lr];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!inf && D0 == 0.0) inf = n;
+    if (act && info) info[s0 + lane] = inf;
+    // back substitution, last chunk first; a system with INFO > 0 keeps its b
+    __threadfence_block();
+    __syncthreads();
+    double x1 = 0.0, x2 = 0.0;  // of rows r + 1 and r + 2
+    const int cl = (n - 1) / kGtRows * kGtRows;
+    load(cl);
+    for (int c0 = cl; c0 >= 0; c0 -= kGtRows) {
+        to_lds();
+        __syncthreads();
+        load(c0 - kGtRows);
+        for (int r = min(kGtRows, n - c0) - 1; r >= 0 && !inf; r--) {
+            const int row = c0 + r;
+            const double Dr = lds[1][lane][r], Br = lds[3][lane][r];
+            double x;
+            if (row == n - 1) x = Br / Dr;
+            else if (row == n - 2) x = (Br - lds[2][lane][r] * x1) / Dr;
+            else x = (Br - lds[2][lane][r] * x1 - lds[0][lane][r] * x2) / Dr;
+            lds[3][lane][r] = x;
+            x2 = x1;
+            x1 = x;
+        }
+        __syncthreads();
+        if (c0 + lr < n) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                const int sys = ls + 64 / kGtRows * q;
+                if (s0 + sys < nsys) b[(s0 + sys) * n + c0 + lr] = lds[3][sys][lr];
+            }
+        }
+        __syncthreads();
+    }
+}
 
 }  // namespace
 
@@ -990,9 +1079,7 @@ void launch_daf_k(hipStream_t s, const Level& L, const Fields& F, const Consts& 
 }
 
 void launch_gtsv_batch(hipStream_t s, int n, int nsys, double* dl, double* d, double* du, double* b, int* info) {
-    const int bs = 64;
-    hipLaunchKernelGGL(k_gtsv_batch, dim3((unsigned)((nsys + bs - 1) / bs)), dim3(bs), 0, s, n, nsys, dl, d, du, b,
-                       info);
+    hipLaunchKernelGGL(k_gtsv_batch, dim3((unsigned)((nsys + 63) / 64)), dim3(64), 0, s, n, nsys, dl, d, du, b, info);
 }
 
 }  // namespace desalm

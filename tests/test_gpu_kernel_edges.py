@@ -140,3 +140,29 @@ def test_state_comes_back_through_the_ring(gpu, dims):
     for s, a in zip(sv, st):
         assert np.array_equal(s.level_field("q"), a[0])
         s.close()
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("n,nsys", [(1, 1), (2, 3), (3, 64), (15, 63), (16, 65), (17, 1), (32, 64), (33, 130),
+                                    (97, 7)])
+def test_gtsv_chunks(gpu, n, nsys, noalloc):
+    """Batched SGTSV at the edges of its 16-row chunks and 64-system waves,
+    with interchanges, and zero pivots at the first, an inner and the last
+    row."""
+    from desalm.lib import gtsv_batch
+    rng = np.random.default_rng(1000 * n + nsys)
+    dl, d, du, b = (rng.uniform(-1, 1, (nsys, n)) for _ in range(4))
+    if nsys >= 3:
+        d[1] = dl[1] = 0.0            # INFO 1
+        d[2, n // 2] = 0.0
+        if n > 1:
+            dl[2, n // 2 - 1] = 0.0   # the row before leaves it zero
+            dl[2, n // 2] = 0.0
+    x, info = gtsv_batch(dl, d, du, b, noalloc=noalloc)
+    for s in range(nsys):
+        xo, io = po.gtsv(dl[s], d[s], du[s], b[s])
+        assert info[s] == io
+        if io == 0:
+            # a solve of random bands: backward stable, so off by a small
+            # multiple of the condition number's share of the largest entry
+            assert np.abs(x[s] - xo).max() <= 1e-9 * max(1.0, np.abs(xo).max())
