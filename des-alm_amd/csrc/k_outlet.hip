@@ -87,7 +87,9 @@ __device__ double diss_aux(const Plane& P, const Fields& F, int j, int k, int d,
     return tmp1 * tmp2;
 }
 
-__global__ void k_outlet_rhs(Level L, Fields F, Consts C, int inout) {
+// one wave per workgroup: a plane is a few thousand nodes, so this spreads it
+// over the CUs and leaves a thread all the registers its gathers need
+__global__ void __launch_bounds__(64) k_outlet_rhs(Level L, Fields F, Consts C, int inout) {
     const int nj = L.nj, nk = L.nk;
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (long)(nj - 2) * (nk - 2)) return;
@@ -250,9 +252,9 @@ __global__ void k_outlet_rhs(Level L, Fields F, Consts C, int inout) {
 
 void launch_outlet_rhs(hipStream_t s, const Level& L, const Fields& F, const Consts& C) {
     const long n = (long)(L.nj - 2) * (L.nk - 2);
-    const unsigned nb = (unsigned)((n + 127) / 128);
-    if (C.btype[0] == DESALM_BC_OUTLET_MOC) hipLaunchKernelGGL(k_outlet_rhs, dim3(nb), dim3(128), 0, s, L, F, C, 1);
-    if (C.btype[1] == DESALM_BC_OUTLET_MOC) hipLaunchKernelGGL(k_outlet_rhs, dim3(nb), dim3(128), 0, s, L, F, C, 2);
+    const unsigned nb = (unsigned)((n + 63) / 64);
+    if (C.btype[0] == DESALM_BC_OUTLET_MOC) hipLaunchKernelGGL(k_outlet_rhs, dim3(nb), dim3(64), 0, s, L, F, C, 1);
+    if (C.btype[1] == DESALM_BC_OUTLET_MOC) hipLaunchKernelGGL(k_outlet_rhs, dim3(nb), dim3(64), 0, s, L, F, C, 2);
 }
 
 }  // namespace desalm
