@@ -322,11 +322,27 @@ void launch_residual(hipStream_t s, const Level& L, const Fields& F, const Const
                      int recalc, int calc_pk, int kc);
 void launch_visc_pk(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int n, int calc_pk, int kc);
 int visc_kc_default(const Level& L);
-// planes per workgroup of a launch over t tiles of one plane each: enough
-// workgroups (about 2048) to fill the chip
-inline int kc_of_tiles(long t) {
-    const long kc = t / 2048;
-    return (int)(kc < 1 ? 1 : kc > 16 ? 16 : kc);
+// planes per workgroup of a marching kernel over t tiles of one plane each,
+// np interior planes.  A workgroup's time goes with kc + 1.5 (its planes and
+// the halo planes it loads first), the launch's with that times the rounds of
+// workgroups that the chip holds at once (per CU: resident): the least product
+// of up to 16 planes.  About 2048 workgroups whatever the round, as before:
+// 97x65x65 one plane, residual 75 us, five planes 66 us; 97x67x65 64 and 60 us,
+// SA update 182 and 168 us; 129^3 305 and 294 us, 573 and 541 us.
+inline int kc_of_tiles(long t, int np, int resident) {
+    if (np < 1) return 1;
+    int best = 1;
+    double cost = 0.0;
+    for (int kc = 1; kc <= 16 && kc <= np; kc++) {
+        const long wg = t / np * ((np + kc - 1) / kc);
+        const long rounds = (wg + 256L * resident - 1) / (256L * resident);
+        const double c = (double)rounds * (kc + 1.5);
+        if (kc == 1 || c < cost) {
+            cost = c;
+            best = kc;
+        }
+    }
+    return best;
 }
 // DAF implicit operator, k_daf.hip
 void launch_daf_i(hipStream_t s, const Level& L, const Fields& F, const Consts& C, int n);

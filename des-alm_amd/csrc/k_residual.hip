@@ -582,7 +582,12 @@ void launch_dtau(hipStream_t s, const Level& L, const Fields& F, const Consts& C
 // tiles of all interior planes of a level
 static long visc_plane_tiles(const Level& L) { return (long)visc_gx(L) * visc_gy(L) * (L.nk - 2); }
 
-int visc_kc_default(const Level& L) { return kc_of_tiles(visc_plane_tiles(L)); }
+// workgroups of k_visc_pk on a CU at once (236 VGPRs, four waves each)
+constexpr int kViscResident = 2;
+
+int visc_kc_default(const Level& L) {
+    return kc_of_tiles(visc_plane_tiles(L), L.nk - 2, kViscResident);
+}
 
 static unsigned node_blocks(const Level& L) { return (unsigned)((L.n + 255) / 256); }
 
@@ -601,9 +606,13 @@ void launch_residual_z(hipStream_t s, const ZoneList& Z, int n, int recalc, int 
     // one plane, whose two halo planes cost every zone: six blocks of 0.16 to
     // 1.3 M nodes, 382 us at one plane, 250 us at nine.)
     if (kc <= 0) {
+        // (t is a mean over the zones' planes times the largest plane count, so
+        // that the rounds are those of the whole launch)
         long t = 0;
+        int np = 1;
+        for (const ZoneDesc& z : Z.host) np = std::max(np, z.lv[n].nk - 2);
         for (const ZoneDesc& z : Z.host) t += visc_plane_tiles(z.lv[n]);
-        kc = kc_of_tiles(t);
+        kc = kc_of_tiles(std::max(1L, t / np) * np, np, kViscResident);
     }
     for (const ZoneDesc& z : Z.host) kc = std::min(kc, z.lv[n].nk - 2);
     unsigned nv = 0;

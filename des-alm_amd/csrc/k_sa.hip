@@ -667,7 +667,12 @@ __global__ void __launch_bounds__(512) k_sa_sweep_z(ZoneGrid G, int P, int TI, i
 
 static long sa_plane_tiles(const Level& L) { return (long)sa_gx(L) * sa_gy(L) * (L.nk - 2); }
 
-int sa_kc_default(const Level& L) { return kc_of_tiles(sa_plane_tiles(L)); }
+// workgroups of k_sa_rhs on a CU at once (168 VGPRs, four waves each)
+constexpr int kSaResident = 3;
+
+int sa_kc_default(const Level& L) {
+    return kc_of_tiles(sa_plane_tiles(L), L.nk - 2, kSaResident);
+}
 
 void launch_sa_prep(hipStream_t s, const Level& L, const Fields& F) {
     const int b = 256;
@@ -747,8 +752,10 @@ void launch_des_eddy_z(hipStream_t s, const ZoneList& Z, int itk, int kc) {
     // the one plane of the smallest of six blocks' own default, 400 us at nine)
     if (kc <= 0) {
         long t = 0;
+        int np = 1;
+        for (const ZoneDesc& z : Z.host) np = std::max(np, z.lv[1].nk - 2);
         for (const ZoneDesc& z : Z.host) t += sa_plane_tiles(z.lv[1]);
-        kc = kc_of_tiles(t);
+        kc = kc_of_tiles(std::max(1L, t / np) * np, np, kSaResident);
     }
     for (const ZoneDesc& z : Z.host) kc = std::min(kc, z.lv[1].nk - 2);
     const ZoneGrid Gq = Z.grid(
