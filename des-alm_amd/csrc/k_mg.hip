@@ -5,12 +5,11 @@
 //   k_nlevel        mg_nlevel: injection of q, xnut, qold_mg and the 27-point
 //                   restriction of rh into pk (src/mg_nlevel.F90:2-150),
 //                   boundary pk zeroed (mg_zero_pk_boundary)
-//   k_prolong_fill  mg_prolong's coarse correction q - qold_mg and its
-//                   k/j/i linear fills onto the fine level
-//                   (src/mg_prolong.F90:57-170), one coarse cell per thread
 //   k_rs_sweep<D>   rs_sweep constant-coefficient smoothing sweeps
-//                   (src/rs_sweep.F90:59-178) with every row on chip,
-//                   k sweep also adds dq to q
+//                   (src/rs_sweep.F90:59-178) with every row on chip; the
+//                   i sweep forms mg_prolong's coarse correction q - qold_mg
+//                   and its k/j/i linear fills (src/mg_prolong.F90:57-170) as
+//                   it loads, the k sweep adds dq to q
 //   k_bc_fm         bcond_fm faces (src/bcond_fm.F90:79-306), k_pfix_*
 //                   the pinned-pressure shift (:310-322)
 //   k_resid_*       mg_residual's L1 update norms (src/mg_residual.F90:58-67)
@@ -116,93 +115,60 @@ struct ProlongCtx {
     int icrs, jcrs, kcrs;
 };
 
-// cells of the fill per direction: a coarsened direction has one cell per
-// pair of adjacent coarse nodes (a, a + 1), with the fine nodes 2a (on coarse
-// node a; interior for a >= 1) and 2a + 1 (between a and a + 1); a direction
-// that is not coarsened has one cell per interior fine node f = a + 1, on
-// coarse node a + 1.  Coarsened directions have odd fine node counts, so
-// 2a + 1 <= nf - 2 for every cell.
-__host__ __device__ inline int fill_cells(int nf, int nc, int crs) { return crs ? nc - 1 : nf - 2; }
-__host__ __device__ inline long fill_cells(const ProlongCtx& P) {
-    return (long)fill_cells(P.Lf.ni, P.Lc.ni, P.icrs) * fill_cells(P.Lf.nj, P.Lc.nj, P.jcrs) *
-           fill_cells(P.Lf.nk, P.Lc.nk, P.kcrs);
-}
-
 // The coarse correction q - qold_mg (mg_prolong.F90:57-75) filled linearly
-// onto the fine level's interior nodes into F.dp, level-local: k, then j,
-// then i (mg_prolong.F90:82-161).  One thread per cell: it loads q and
-// qold_mg at the cell's eight coarse corners once and forms each of its (up
-// to eight) fine nodes from them.  A fine node coincident with a coarse node
-// in a direction takes the low corner there (the reference's high and low
-// nodes are then the same node), one between two coarse nodes takes half of
-// each: the same operands in the same order as the reference's fills.
-__device__ __forceinline__ void prolong_fill_body(const ProlongCtx& P, const Fields& F, unsigned bid, unsigned nb) {
-    const Level& Lf = P.Lf;
+// onto R fine nodes i = s0 + 1 .. of the line (jf, kf) for the i sweep: k, then
+// j, then i (mg_prolong.F90:82-161).  A fine node coincident with a coarse node
+// in a direction takes it, one between two coarse nodes takes half of each: the
+// same operands in the same order as the reference's fills (halves are exact,
+// so the order alone fixes the bits).  The sweep reads the coarse nodes
+// straight (an eighth as many, shared by neighbouring lines in L2) instead of
+// a filled field that a launch of its own wrote: prolongation 197 -> 188 us on
+// 193x129x129, and one launch less per level.
+template <int R>
+__device__ __forceinline__ void fill_rows(const ProlongCtx& P, const Fields& F, int jf, int kf, int s0, double (&w)[R][4]) {
     const Level& Lc = P.Lc;
-    const int ca = fill_cells(Lf.ni, Lc.ni, P.icrs), cb = fill_cells(Lf.nj, Lc.nj, P.jcrs);
-    const long t = (long)xcd_block(bid, nb) * blockDim.x + threadIdx.x;
-    if (t >= fill_cells(P)) return;
-    const int a = (int)(t % ca), b = (int)((t / ca) % cb), c = (int)(t / ((long)ca * cb));
-    // per direction: low and high coarse corner, fine index of node 0, and
-    // whether nodes 0 (coincident) and 1 (between) exist
-    const int cl[3] = {P.icrs ? a : a + 1, P.jcrs ? b : b + 1, P.kcrs ? c : c + 1};
-    const int crs[3] = {P.icrs, P.jcrs, P.kcrs};
-    int ch[3], f0[3];
-    bool has0[3], has1[3];
+    const bool jodd = P.jcrs && (jf & 1), kodd = P.kcrs && (kf & 1);
+    const int jl = P.jcrs ? jf >> 1 : jf, kl = P.kcrs ? kf >> 1 : kf;
+    const long sJ = Lc.ni, sK = (long)Lc.ni * Lc.nj;
+    const long line = Lc.off + sJ * jl + sK * kl;
+    // coarse node c of the row, j and k filled
+    auto node = [&](int c, double (&f)[4]) {
+        const long l = line + min(c, Lc.ni - 1);
+        auto corr = [&](long g, double (&v)[4]) {
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        ch[d] = crs[d] ? cl[d] + 1 : cl[d];
-        f0[d] = crs[d] ? 2 * cl[d] : cl[d];
-        has0[d] = !crs[d] || cl[d] >= 1;
-        has1[d] = crs[d];
-    }
-    long corner[2][2][2];  // [i side][j side][k side], side 1 = high
+            for (int m = 0; m < 4; m++) v[m] = F.q[m][g] - F.qold[m][g];
+        };
+        auto kfill = [&](long g, double (&v)[4]) {
+            corr(g, v);
+            if (kodd) {
+                double h[4];
+                corr(g + sK, h);
 #pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++)
-#pragma unroll
-            for (int z = 0; z < 2; z++)
-                corner[x][y][z] = Lc.off + lidx(Lc, x ? ch[0] : cl[0], y ? ch[1] : cl[1], z ? ch[2] : cl[2]);
-    const long base = lidx(Lf, f0[0], f0[1], f0[2]);
-    const long sI = 1, sJ = Lf.ni, sK = (long)Lf.ni * Lf.nj;
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        double v[2][2][2];
-#pragma unroll
-        for (int x = 0; x < 2; x++)
-#pragma unroll
-            for (int y = 0; y < 2; y++)
-#pragma unroll
-                for (int z = 0; z < 2; z++) {
-                    const long l = corner[x][y][z];
-                    v[x][y][z] = F.q[m][l] - F.qold[m][l];
-                }
-        // fk[x][y][pk]: the k fill of node parity pk on the (x, y) corner column
-        double fk[2][2][2];
-#pragma unroll
-        for (int x = 0; x < 2; x++)
-#pragma unroll
-            for (int y = 0; y < 2; y++) {
-                fk[x][y][0] = v[x][y][0];
-                fk[x][y][1] = 0.5 * v[x][y][1] + 0.5 * v[x][y][0];
+                for (int m = 0; m < 4; m++) v[m] = 0.5 * h[m] + 0.5 * v[m];
             }
+        };
+        kfill(l, f);
+        if (jodd) {
+            double h[4];
+            kfill(l + sJ, h);
 #pragma unroll
-        for (int pk = 0; pk < 2; pk++) {
-            if (!(pk ? has1[2] : has0[2])) continue;
-#pragma unroll
-            for (int pj = 0; pj < 2; pj++) {
-                if (!(pj ? has1[1] : has0[1])) continue;
-                double fj[2];
-#pragma unroll
-                for (int x = 0; x < 2; x++) fj[x] = pj ? 0.5 * fk[x][1][pk] + 0.5 * fk[x][0][pk] : fk[x][0][pk];
-#pragma unroll
-                for (int pi = 0; pi < 2; pi++) {
-                    if (!(pi ? has1[0] : has0[0])) continue;
-                    F.dp[m][base + pi * sI + pj * sJ + pk * sK] = pi ? 0.5 * fj[1] + 0.5 * fj[0] : fj[0];
-                }
-            }
+            for (int m = 0; m < 4; m++) f[m] = 0.5 * h[m] + 0.5 * f[m];
         }
+    };
+    if (P.icrs) {
+        // rows i = s0 + 1 (between), s0 + 2 (coincident), ...: coarse nodes
+        // s0 / 2 .. (s0 + R) / 2 (s0 and R are even)
+        double f[R / 2 + 1][4];
+#pragma unroll
+        for (int u = 0; u <= R / 2; u++) node(s0 / 2 + u, f[u]);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+                w[r][m] = r % 2 == 0 ? 0.5 * f[r / 2 + 1][m] + 0.5 * f[r / 2][m] : f[r / 2 + 1][m];
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) node(s0 + 1 + r, w[r]);
     }
 }
 
@@ -212,8 +178,9 @@ __device__ __forceinline__ void prolong_fill_body(const ProlongCtx& P, const Fie
 // D = 2 adds the result to q instead.  The reference calls SGTSV with four
 // right-hand sides; this is its non-interchanging elimination.
 template <int D, int R>
-__device__ __forceinline__ void rs_sweep_body(const Level& L, const Fields& F, const SegShape& sh, double epn,
+__device__ __forceinline__ void rs_sweep_body(const ProlongCtx& PC, const Fields& F, const SegShape& sh, double epn,
                                               unsigned bid) {
+    const Level& L = PC.Lf;
     extern __shared__ double smem_rs[];
     const int P = sh.P, TI = sh.TI, n = sh.n;
     const int tid = (int)threadIdx.x;
@@ -244,26 +211,13 @@ __device__ __forceinline__ void rs_sweep_body(const Level& L, const Fields& F, c
         c[r] = -epn;
     }
     if (D == 0) {
-        // i lines: the R rows are one run of consecutive nodes, loaded as
-        // such (16-byte loads; lanes are R rows apart).  A partial last
-        // segment loads the line's last R rows and shifts them into place.
-        const int pb = max(0, min(s0, n - R));
-        const int shift = s0 - pb;
+        // i lines: the coarse correction, filled here
         double w[R][4];
+        fill_rows<R>(PC, F, act ? (int)(1 + t % (nj - 2)) : 1, act ? (int)(1 + t / (nj - 2)) : 1, s0, w);
 #pragma unroll
         for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int m = 0; m < 4; m++) w[r][m] = F.dp[m][base + pb + r + 1];
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                double v = w[r][m];
-#pragma unroll
-                for (int t = 1; t < R; t++)
-                    if (shift == t) v = r + t < R ? w[r + t < R ? r + t : R - 1][m] : 0.0;
-                d[r][m] = r < nr ? v : 0.0;
-            }
+            for (int m = 0; m < 4; m++) d[r][m] = r < nr ? w[r][m] : 0.0;
     } else {
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -647,27 +601,17 @@ __global__ void __launch_bounds__(256) k_nlevel_z(ZoneGrid G, int n) {
     const int ic = Z.icrs, jc = Z.jcrs, kc = Z.kcrs;
     nlevel_body(Lc, Lf, F, ic, jc, kc, b.bid, b.nblk);
 }
-__global__ void __launch_bounds__(256) k_prolong_fill(ProlongCtx P, Fields F) {
-    prolong_fill_body(P, F, blockIdx.x, gridDim.x);
-}
-__global__ void __launch_bounds__(256) k_prolong_fill_z(ZoneGrid G, int n) {
-    const ZoneBlock b = zone_block(G);
-    const ZoneDesc& Z = G.z[b.z];
-    const ProlongCtx P{Z.lv[n], Z.lv[n + 1], Z.icrs, Z.jcrs, Z.kcrs};
-    const Fields F = Z.F;
-    prolong_fill_body(P, F, b.bid, b.nblk);
-}
 template <int D, int R>
-__global__ void __launch_bounds__(512) k_rs_sweep(Level L, Fields F, SegShape sh, double epn) {
-    rs_sweep_body<D, R>(L, F, sh, epn, xcd_block(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(512) k_rs_sweep(ProlongCtx P, Fields F, SegShape sh, double epn) {
+    rs_sweep_body<D, R>(P, F, sh, epn, xcd_block(blockIdx.x, gridDim.x));
 }
 template <int D, int R>
 __global__ void __launch_bounds__(512) k_rs_sweep_z(ZoneGrid G, int n, int P, int TI) {
     const ZoneBlock b = zone_block(G);
     const ZoneDesc& Z = G.z[b.z];
-    const Level L = Z.lv[n];
+    const ProlongCtx PC{Z.lv[n], Z.lv[n + 1], Z.icrs, Z.jcrs, Z.kcrs};
     const Fields F = Z.F;
-    rs_sweep_body<D, R>(L, F, seg_lines(L, D, P, TI), Z.C.ep[1][D], xcd_block(b.bid, b.nblk));
+    rs_sweep_body<D, R>(PC, F, seg_lines(PC.Lf, D, P, TI), Z.C.ep[1][D], xcd_block(b.bid, b.nblk));
 }
 template <int E0, int E1>
 __global__ void __launch_bounds__(256) k_bc_fm(Level L, Fields F, Consts C, long nfix) {
@@ -728,7 +672,8 @@ void launch_zero_pk_boundary(hipStream_t s, const Level& L, const Fields& F) {
 
 // the smoothing sweep of direction D over the interior lines of level L
 template <int D>
-static void rs_sweep(hipStream_t s, const Level& L, const Fields& F, double ep) {
+static void rs_sweep(hipStream_t s, const ProlongCtx& P, const Fields& F, double ep) {
+    const Level& L = P.Lf;
     const int n = D == 0 ? L.ni - 2 : D == 1 ? L.nj - 2 : L.nk - 2;
     const long nl = D == 0 ? (long)(L.nj - 2) * (L.nk - 2) : D == 1 ? (long)(L.ni - 2) * (L.nk - 2)
                                                                     : (long)(L.ni - 2) * (L.nj - 2);
@@ -739,18 +684,17 @@ static void rs_sweep(hipStream_t s, const Level& L, const Fields& F, double ep) 
     const unsigned nb = (unsigned)((sh.nlines + sh.TI - 1) / sh.TI);
     const size_t lds = seg_lds_bytes(sh, 4);
     if (R == 4)
-        hipLaunchKernelGGL((k_rs_sweep<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, sh, ep);
+        hipLaunchKernelGGL((k_rs_sweep<D, 4>), dim3(nb), dim3(sh.TI * sh.P), lds, s, P, F, sh, ep);
     else
-        hipLaunchKernelGGL((k_rs_sweep<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, L, F, sh, ep);
+        hipLaunchKernelGGL((k_rs_sweep<D, 8>), dim3(nb), dim3(sh.TI * sh.P), lds, s, P, F, sh, ep);
 }
 
 void launch_prolong(hipStream_t s, const Level& Lf, const Level& Lc, const Fields& F, const Consts& C, int icrs,
                     int jcrs, int kcrs) {
     ProlongCtx P{Lf, Lc, icrs, jcrs, kcrs};
-    hipLaunchKernelGGL(k_prolong_fill, dim3(nblk(fill_cells(P), 256)), dim3(256), 0, s, P, F);
-    rs_sweep<0>(s, Lf, F, C.ep[1][0]);
-    rs_sweep<1>(s, Lf, F, C.ep[1][1]);
-    rs_sweep<2>(s, Lf, F, C.ep[1][2]);
+    rs_sweep<0>(s, P, F, C.ep[1][0]);
+    rs_sweep<1>(s, P, F, C.ep[1][1]);
+    rs_sweep<2>(s, P, F, C.ep[1][2]);
 }
 
 void launch_outlet_ratios(hipStream_t s, const Level& L, const Fields& F, const int* btype, const int* bdir) {
@@ -860,11 +804,6 @@ static void rs_sweep_z(hipStream_t s, const ZoneList& Z, int n) {
 
 // prolongation from level n + 1 onto level n
 void launch_prolong_z(hipStream_t s, const ZoneList& Z, int n) {
-    unsigned nf = 0;
-    const ZoneGrid Gf = Z.grid(
-        [&](const ZoneDesc& z) { return nblk(fill_cells(ProlongCtx{z.lv[n], z.lv[n + 1], z.icrs, z.jcrs, z.kcrs}), 256); },
-        nf);
-    hipLaunchKernelGGL(k_prolong_fill_z, dim3(nf), dim3(256), 0, s, Gf, n);
     rs_sweep_z<0>(s, Z, n);
     rs_sweep_z<1>(s, Z, n);
     rs_sweep_z<2>(s, Z, n);
