@@ -44,14 +44,15 @@ __device__ __forceinline__ void st32(T* a, unsigned idx, T v) {
     *reinterpret_cast<T*>(reinterpret_cast<char*>(a) + idx * (unsigned)sizeof(T)) = v;
 }
 
-// FP64 division, reciprocal, reciprocal square root and square root from the
+// FP64 division, reciprocal and square root with its reciprocal from the
 // hardware estimates, for normal operands (a zero divisor or an infinite
-// operand gives NaN, a zero radicand an infinite reciprocal root and a zero
-// root).  One Newton step takes the ~2^-23 reciprocal estimate to ~2^-46 and
-// the residual step of the quotient, or a second Newton step, leaves about the
-// final rounding alone; the root's third-order step goes there at once.  Half
-// the instructions of the IEEE sequences, which also scale and fix up every
-// special case.
+// operand gives NaN, a zero radicand a zero root and an infinite reciprocal).
+// One Newton step takes the ~2^-23 reciprocal estimate to ~2^-46, and the
+// residual step of the quotient, or a second Newton step, is off by ~2^-91
+// before its rounding: the correctly rounded value but for one operand in
+// ~2^38, so results keep the bits of the IEEE operations.  Half the
+// instructions of their sequences, which also scale and fix up every special
+// case.
 __device__ __forceinline__ double div64(double a, double b) {
     double r = __builtin_amdgcn_rcp(b);
     r = fma(r, fma(-b, r, 1.0), r);
@@ -63,17 +64,17 @@ __device__ __forceinline__ double rcp64(double b) {
     r = fma(r, fma(-b, r, 1.0), r);
     return fma(r, fma(-b, r, 1.0), r);
 }
-__device__ __forceinline__ double rsqrt64(double x) {
+// s = sqrt(x) and is = 1 / s, both rounded as the two IEEE operations: a
+// third-order step on the estimate of 1 / sqrt(x), the root's residual step,
+// and a Newton step to the reciprocal of the rounded root
+__device__ __forceinline__ void root64(double x, double& s, double& is) {
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma(-(x * y), y, 1.0);
     const double r = fma(y * e, fma(0.375, e, 0.5), y);
-    return x == 0.0 ? y : r;
-}
-// sqrt(x) given y = rsqrt64(x)
-__device__ __forceinline__ double sqrt64(double x, double y) {
-    const double s = x * y;
-    const double r = fma(fma(-s, s, x), 0.5 * y, s);
-    return x == 0.0 ? 0.0 : r;
+    const double t = x * r;
+    const double q = fma(fma(-t, t, x), 0.5 * r, t);
+    s = x == 0.0 ? 0.0 : q;
+    is = x == 0.0 ? y : fma(r, fma(-q, r, 1.0), r);
 }
 // 1 / x in the type of a line solve
 __device__ __forceinline__ double recip(double x) { return rcp64(x); }

@@ -45,8 +45,9 @@ namespace {
 // beta / sigma (rhs_modal_matrices.F90:82-84)
 //
 // The FP64 form takes reciprocals and roots from the hardware estimates
-// (rcp64 and its like; errors of 0.5 ulp, 1 ulp for the reciprocal root, as
-// the IEEE operations they stand for).  The sweeps spent up to half their time
+// (rcp64 and its like, correctly rounded as the IEEE operations they stand for
+// but for rare operands).  Roots to 1 ulp only moved the solution by rounding,
+// and a network trained on such solutions by 1e-8 of its loss.  The sweeps spent up to half their time
 // issuing instructions, two fifths of them divisions and roots: with these and
 // the scaling of maps and the divisions of the c' scan moved out of its serial
 // chain, i 124 -> 110 us, j 120 -> 109 us, k 150 -> 142 us on 193x129x129 and
@@ -57,15 +58,16 @@ namespace {
 template <typename S>
 struct Num {  // S = double
     static __device__ __forceinline__ double rcp(double x) { return rcp64(x); }
+    static __device__ __forceinline__ double div(double a, double b) { return div64(a, b); }
     // sqrt(x) and 1 / sqrt(x)
     static __device__ __forceinline__ void root(double x, double& s, double& is) {
-        is = rsqrt64(x);
-        s = sqrt64(x, is);
+        root64(x, s, is);
     }
 };
 template <>
 struct Num<float> {
     static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+    static __device__ __forceinline__ double div(double a, double b) { return a / b; }
     static __device__ __forceinline__ void root(double x, double& s, double& is) {
         s = sqrt(x);
         is = 1.0 / s;
@@ -79,8 +81,7 @@ template <typename S>
 __device__ __forceinline__ NodeDt node_dt(const Consts& C, double dt) {
     NodeDt n;
     n.dt = dt;
-    if (sizeof(S) == 8) n.alpha = 1.0 + C.e_source * 1.5 / C.delti * dt;
-    else n.alpha = 1.0 + C.e_source * 1.5 * dt / C.delti;
+    n.alpha = 1.0 + Num<S>::div(C.e_source * 1.5 * dt, C.delti);
     Num<S>::root(C.beta * n.alpha, n.sigma, n.isigma);
     n.theta = C.beta * n.isigma;
     return n;
@@ -395,12 +396,13 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
         // j and k lines: the loads of window entry w + 1 are in flight while
         // entry w is transformed, at addresses clamped to the line (no branch,
         // which would hold back the next row's loads; all rows' loads at once
-        // would not fit the registers)
+        // would not fit the registers).  The last entry is the node after the
+        // segment's rows, wherever they end.
         struct In {
             double dt, a[3], m[3], x[4];
         };
         auto load = [&](int w, In& o) {
-            const long tl = base + (long)min(s0 + w, nd - 1) * sD, g = L.off + tl;
+            const long tl = base + (long)min(w <= R ? s0 + w : pe, nd - 1) * sD, g = L.off + tl;
             o.dt = F.dtau[g];
             metric_row<D>(F, g, o.m[0], o.m[1], o.m[2]);
             if (w >= 1 && w <= R) {
@@ -419,12 +421,19 @@ __device__ __forceinline__ void daf_body(const Level& L, const Fields& F, const 
                 const bool in = w - 1 < nr;
                 double v[4] = {cur.x[0], cur.x[1], cur.x[2], cur.x[3]};
                 const double sd = transform_vals<D, S>(nd0, cur.a, cur.m, v);
-                sdv[w] = (in || (w == nr + 1 && nr > 0)) ? (S)sd : S(0);
+                sdv[w] = in ? (S)sd : S(0);
 #pragma unroll
                 for (int m = 0; m < 4; m++) dv[w - 1][m] = in ? (S)v[m] : S(0);
             } else {
-                const double sd = sd_vals<S>(nd0, cur.m);
-                sdv[w] = (w == 0 ? nr > 0 : nr == R) ? (S)sd : S(0);
+                const S sd = (S)sd_vals<S>(nd0, cur.m);
+                if (w == 0) {
+                    sdv[0] = nr > 0 ? sd : S(0);
+                } else {
+                    sdv[R + 1] = S(0);
+#pragma unroll
+                    for (int q = 1; q <= R + 1; q++)
+                        if (q == nr + 1 && nr > 0 && pe <= nd - 1) sdv[q] = sd;
+                }
             }
             cur = nxt;
         }
