@@ -47,9 +47,9 @@ namespace {
 // The FP64 form takes reciprocals and roots from the hardware estimates
 // (rcp64 and its like, correctly rounded as the IEEE operations they stand for
 // but for rare operands).  Roots to 1 ulp only moved the solution by rounding,
-// and a network trained on such solutions by 1e-8 of its loss.  The sweeps spent up to half their time
-// issuing instructions, two fifths of them divisions and roots: with these and
-// the scaling of maps and the divisions of the c' scan moved out of its serial
+// and a network trained on such solutions by 1e-8 of its loss.  The sweeps
+// spent up to half their time issuing instructions, two fifths of them
+// divisions and roots: with these and the scaling of maps and the divisions of the c' scan moved out of its serial
 // chain, i 124 -> 110 us, j 120 -> 109 us, k 150 -> 142 us on 193x129x129 and
 // 15.7 -> 12.4 us for the k sweep of 49x33x33, where the chain is all there is.
 // The FP32 form keeps the IEEE operations: its solves amplify any difference

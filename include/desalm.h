@@ -364,7 +364,8 @@ int64_t desalm_device_bytes(const desalm_ctx* ctx);
 
 /* Launch shape of the LDS-tiled stencil kernels: k planes per workgroup of
  * the viscous kernel on each level (kc_visc[0 .. ng-1]) and of the SA
- * right-hand side (fine level); 0 picks the default (about 2048 workgroups).
+ * right-hand side (fine level); 0 picks the default (the fewest rounds of
+ * workgroups, weighed against the planes each marches).
  * The shape changes results only by rounding (where a workgroup's first k
  * face is evaluated, multiply-adds may be contracted differently).
  * desalm_autotune times every candidate
