@@ -983,6 +983,7 @@ int desalm_mg_driver(desalm_ctx* c, int* itc_out, double* resid_out) {
     }
     HIPCHK(c, hipEventRecord(c->ev1, s));
     HIPCHK(c, hipStreamSynchronize(s));
+    prof_flush(c);  // the launches after the last pseudo-iteration
     float ms = 0.0f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;
@@ -1507,6 +1508,7 @@ int desalm_group_mg_driver(desalm_group* g, int* itc_out, double* resid_out) {
     if (!rc) rc = vcycles(g->z, g->nd > 0, g->mom, exchange, g->init_resd, itc_out, resid_out, batch ? &g->zl : nullptr);
     if (!rc && hipEventRecord(g->ev1, s) != hipSuccess) rc = fail(c0, "hipEventRecord failed");
     if (hipStreamSynchronize(s) != hipSuccess && !rc) rc = fail(c0, "hipStreamSynchronize failed");
+    for (desalm_ctx* c : g->z) prof_flush(c);  // the launches after the last pseudo-iteration
     for (size_t z = 0; z < g->z.size(); z++) g->z[z]->stream = own[z];
     if (rc) return rc;
     float ms = 0.0f;
