@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "desalm_internal.h"
+#include "host_copy.h"
 
 using namespace desalm;
 

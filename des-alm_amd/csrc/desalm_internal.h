@@ -304,12 +304,6 @@ struct ZoneList {
     }
 };
 
-// host_copy.hip: copy from device memory to pageable host memory, after the
-// work on s, complete on return; and the number of contexts that keep its
-// pinned ring alive
-hipError_t host_read(void* dst, const void* src, size_t bytes, hipStream_t s, int device);
-void host_read_users(int change);
-
 // ---- launchers (each enqueues on `s`) ----
 // residual assembly, k_residual.hip
 // dtau and fv of level n; on a fine level with a characteristic outlet also

@@ -6,22 +6,24 @@
 // it in chunks through a pinned ring instead; the DMA of the next chunks runs
 // while several threads copy the chunks that have arrived.  128 MB (q of a
 // 193x129x129 block) into fresh pages: 11.9 -> 3.7 ms with four threads (two: 5.9,
-// eight: 3.4; 3.3 is the link).
+// eight: 3.4; 3.3 is the link).  The count does not follow the caller's CPU
+// affinity: the four threads of a process held to two CPUs take 6.1 ms, to one
+// 10.1 ms (resident pages 4.2 and 5.0), a plain copy there 12.4 ms (7.4).
 // Host-to-device copies are left to the runtime (30 GB/s).
 //
 // The ring is the process's: kSlots chunks of pinned memory, allocated by the
-// first large read, used by one read at a time (a mutex), and freed when the
-// last context is finalized (a program without contexts, which may read
-// through desalm_gtsv_batch, keeps its 16 MiB until it ends).
+// first large read, used by one read at a time (a mutex, taken once the read's
+// stream is idle), and freed when the last context is finalized (a program
+// without contexts, which may read through desalm_gtsv_batch, keeps its 16 MiB
+// until it ends).
 #include <string.h>
 
 #include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <thread>
-#include <vector>
 
-#include "desalm_internal.h"
+#include "host_copy.h"
 
 namespace desalm {
 
@@ -69,6 +71,11 @@ hipError_t host_read(void* dst, const void* src, size_t bytes, hipStream_t s, in
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     };
     if (bytes < kSmall) return plain();
+    // the stream's earlier work is waited for outside the lock, which then
+    // covers the copy alone: a read behind pending kernels does not hold up
+    // reads of other contexts or the end of one
+    const hipError_t before = hipStreamSynchronize(s);
+    if (before != hipSuccess) return before;
     std::lock_guard<std::mutex> lock(g_mutex);
     if (!g_ring && hipHostMalloc((void**)&g_ring, kSlots * kChunk, hipHostMallocPortable) != hipSuccess) {
         g_ring = nullptr;
