@@ -63,6 +63,17 @@ void copy_chunks(int w, int device, char* dst, const char* src, size_t bytes, hi
     }
 }
 
+// Pinned, managed or device memory: the DMA writes it in place (128 MB into
+// pinned memory 2.36 ms, through the ring 3.28).
+bool known_to_runtime(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 }  // namespace
 
 hipError_t host_read(void* dst, const void* src, size_t bytes, hipStream_t s, int device) {
@@ -70,7 +81,7 @@ hipError_t host_read(void* dst, const void* src, size_t bytes, hipStream_t s, in
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     };
-    if (bytes < kSmall) return plain();
+    if (bytes < kSmall || known_to_runtime(dst)) return plain();
     // the stream's earlier work is waited for outside the lock, which then
     // covers the copy alone: a read behind pending kernels does not hold up
     // reads of other contexts or the end of one

@@ -73,3 +73,15 @@ def test_read_does_not_wait_for_another_streams_work(hc):
     t[1].join(30)
     assert done
     assert all(np.array_equal(d, s) for d, s in zip(dst, src))
+
+
+def test_memory_the_runtime_knows_is_copied_into_directly(hc):
+    """Pinned (or any other registered) destinations take one copy and no
+    pass through the ring."""
+    src = np.random.default_rng(7).standard_normal(LARGE)
+    dst = np.zeros(LARGE)
+    hc.hc_know(dst.ctypes.data)
+    hc.hc_direct()
+    read(hc, dst, src)
+    assert np.array_equal(dst, src)
+    assert hc.hc_direct() == 1
