@@ -45,24 +45,24 @@ __device__ __forceinline__ void st32(T* a, unsigned idx, T v) {
 }
 
 // FP64 division, reciprocal and square root with its reciprocal from the
-// hardware estimates, for normal operands (a zero divisor or an infinite
-// operand gives NaN, a zero radicand a zero root and an infinite reciprocal).
-// One Newton step takes the ~2^-23 reciprocal estimate to ~2^-46, and the
-// residual step of the quotient, or a second Newton step, is off by ~2^-91
-// before its rounding: the correctly rounded value but for one operand in
-// ~2^38, so results keep the bits of the IEEE operations.  Half the
-// instructions of their sequences, which also scale and fix up every special
-// case.
+// hardware estimates.  One Newton step takes the ~2^-23 reciprocal estimate to
+// ~2^-46, and the residual step of the quotient, or a second Newton step, is
+// off by ~2^-91 before its rounding: the correctly rounded value but for one
+// operand in ~2^38, so results keep the bits of the IEEE operations.  About
+// half the instructions of their sequences, which also rescale operands whose
+// quotient or intermediates leave the normal range; these do not (operands and
+// results within 2^-960 .. 2^960 in magnitude).  Zero, infinite and NaN
+// operands give what the IEEE operations give.
 __device__ __forceinline__ double div64(double a, double b) {
     double r = __builtin_amdgcn_rcp(b);
     r = fma(r, fma(-b, r, 1.0), r);
     const double q = a * r;
-    return fma(fma(-b, q, a), r, q);
+    return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), r, q), b, a);
 }
 __device__ __forceinline__ double rcp64(double b) {
     double r = __builtin_amdgcn_rcp(b);
     r = fma(r, fma(-b, r, 1.0), r);
-    return fma(r, fma(-b, r, 1.0), r);
+    return __builtin_amdgcn_div_fixup(fma(r, fma(-b, r, 1.0), r), b, 1.0);
 }
 // s = sqrt(x) and is = 1 / s, both rounded as the two IEEE operations: a
 // third-order step on the estimate of 1 / sqrt(x), the root's residual step,
@@ -73,8 +73,9 @@ __device__ __forceinline__ void root64(double x, double& s, double& is) {
     const double r = fma(y * e, fma(0.375, e, 0.5), y);
     const double t = x * r;
     const double q = fma(fma(-t, t, x), 0.5 * r, t);
-    s = x == 0.0 ? 0.0 : q;
-    is = x == 0.0 ? y : fma(r, fma(-q, r, 1.0), r);
+    const bool special = __builtin_amdgcn_class(x, 0x260);  // -0, +0, +inf
+    s = special ? x : q;
+    is = special ? y : fma(r, fma(-q, r, 1.0), r);
 }
 // 1 / x in the type of a line solve
 __device__ __forceinline__ double recip(double x) { return rcp64(x); }
