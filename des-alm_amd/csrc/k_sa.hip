@@ -361,7 +361,9 @@ __device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, con
             r = r + s_fc[1][ty][tx] - s_fc[1][ty - 1][tx];
             r = r + fkc1 - fkc;
             const double dtjb = 2.0 * C.delti * aj;
-            const double dq5dt = C.e_source * qdiv(3.0 * q(0, 0, 0) - 4.0 * qn5 + qnm15, dtjb);
+            // (with the division fix-up: zero for an infinite time step)
+            const double dq5 = 3.0 * q(0, 0, 0) - 4.0 * qn5 + qnm15;
+            const double dq5dt = C.e_source * __builtin_amdgcn_div_fixup(qdiv(dq5, dtjb), dtjb, dq5);
             r = r + dq5dt - visc - qdiv(psa, aj);
             st32(F.rh5, (unsigned)(t), -dtev * aj * r);
             st32(F.dtj, (unsigned)(t), 0.5 * dtev * aj);

@@ -27,7 +27,7 @@ def test_oracle_takes_an_infinite_time_step(des, unsteady):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("des", [False])
+@pytest.mark.parametrize("des", [False, True])
 @pytest.mark.parametrize("unsteady", [False, True])
 @pytest.mark.parametrize("prec", [0, 1])
 def test_infinite_time_step(gpu, des, unsteady, prec):
