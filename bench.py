@@ -35,7 +35,9 @@ HBM_PEAK_GBS = 8000.0
 
 # compulsory FP64 words per node of the level, per launch (reads + writes):
 # each live input array read once and each output written once, the
-# library's scratch arrays excluded
+# library's scratch arrays excluded.  des_eddy and prolong are chains of
+# launches that meet in scratch arrays (the right-hand side of their sweeps):
+# theirs are the arrays that each launch of the chain reads and writes.
 WORDS = {
     "dtau": 9 + 1 + 1,                        # metrics, xnut -> dtau
     "residual": 4 + 9 + 1 + 1 + 3 + 3 + 1 + 4 + 1,   # q,metrics,aj,xnut,qn,qnm1,dtau -> rh,diss1 (fine)
@@ -43,17 +45,18 @@ WORDS = {
     "daf_i": 4 + 1 + 1 + 3 + 4,               # rh,dtau,aj,csi -> rh
     "daf_j": 4 + 1 + 3 + 3 + 4,               # rh,dtau,csi,eta -> rh
     "daf_k": 4 + 1 + 3 + 3 + 4 + 4,           # rh,dtau,eta,zet,q -> q
-    # des_eddy, per call: itk x (explicit SA rhs + update 22 words, three ADI
-    # sweeps 11 words each) + vorticity source once (13 words); itk applied below
+    # des_eddy, per call: vorticity and contravariant velocities (13 -> 4), itk x
+    # (right-hand side 19 -> 5, i and j sweeps 4 -> 1 each, k sweep with the
+    # update 6 -> 1), nu~ floor and nu_t once (1 -> 2); itk applied below
     "des_eddy": None,
-    "prolong": 33,                            # coarse q, qold, q, dq of the three smoothing sweeps
+    "prolong": 1 + 4 + (4 + 4) + (8 + 4),     # coarse q, qold -> dq (i), dq -> dq (j), dq, q -> q (k)
     "resid_norm": 16,                         # q, qold -> qold (L1 norms), p (pinned-pressure shift)
 }
 
 
 def level_words(name, n, itk=2):
     if name == "des_eddy":
-        return itk * (22 + 3 * 11) + 13
+        return (13 + 4) + itk * ((19 + 5) + 2 * (4 + 1) + (6 + 1)) + (1 + 2)
     w = WORDS[name]
     if name == "residual" and n > 1:
         w += 4 + 4  # pk read and (first pass) written
