@@ -49,12 +49,16 @@ namespace {
 // but for rare operands).  Roots to 1 ulp only moved the solution by rounding,
 // and a network trained on such solutions by 1e-8 of its loss.  The sweeps
 // spent up to half their time issuing instructions, two fifths of them
-// divisions and roots: with these and the scaling of maps and the divisions of the c' scan moved out of its serial
-// chain, i 124 -> 110 us, j 120 -> 109 us, k 150 -> 142 us on 193x129x129 and
-// 15.7 -> 12.4 us for the k sweep of 49x33x33, where the chain is all there is.
-// The FP32 form keeps the IEEE operations: its solves amplify any difference
+// divisions and roots: with these, and with the scaling of maps and the
+// divisions of the c' scan moved out of its serial chain, i 124 -> 110 us,
+// j 120 -> 109 us, k 150 -> 142 us on 193x129x129 and 15.7 -> 12.4 us for the
+// k sweep of 49x33x33, where the chain is all there is.
+// The FP32 form keeps the IEEE operations.  Its solves amplify any difference
 // of the transformed rows (one ulp of FP64 changes which FP32 value a row
-// rounds to), so its results would move by 1e-9 with nothing gained.
+// rounds to), to 1e-9 of the solution within some thirty iterations, and
+// although the helpers round as IEEE does, the compiler contracts the
+// arithmetic around them otherwise: the FP64 form moved by rounding on
+// curvilinear grids when it took them.
 template <typename S>
 struct Num {  // S = double
     static __device__ __forceinline__ double rcp(double x) { return rcp64(x); }

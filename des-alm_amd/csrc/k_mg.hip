@@ -302,10 +302,14 @@ __global__ void k_outlet_ratio(Level L, Fields F, int b, int dir) {
 // before.  One launch does all three: the value a node has after direction E
 // is formed from the values its one or two source nodes have after direction
 // E - 1, down to nodes that no face writes (bc_value), and a node is stored by
-// the thread of its last direction alone.  The nodes read from memory are
-// written by no thread: a source of direction E lies one or two nodes off that
-// face, and a source on a later direction's face belongs to a node that the
-// later direction overwrites.  (Three launches in sequence: 15 us on a level
+// the thread of its last direction alone.  A node that another thread's chain
+// reads from memory is stored by no thread (a node inside the block), or its
+// own chain is the identity in every component that the reader uses: faces of
+// types 0 and 5, type 8 but on the high i face, i faces of type 6, the source
+// plane of a two-sided copy, the velocities of an inflow face.  Its owner
+// stores such a component with the bits it read, so the reader gets the same
+// from before and after that store; a rule that would change one needs a
+// launch of its own.  (Three launches in sequence: 15 us on a level
 // of 33^3 nodes, where each is little more than its launch; 8.4 us in one.)
 // Exception: a plane copy (btype 6) on one face of a direction only reads the
 // opposite plane that its own rule overwrites; then every direction has its

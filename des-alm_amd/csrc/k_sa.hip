@@ -397,9 +397,11 @@ __device__ __forceinline__ void sa_rhs_body(const Level& L, const Fields& F, con
 // rhs_sa_bcond faces (rhs_sa_bcond.F90:40-269): i, then j, then k, in one
 // launch as bcond_fm's are (k_mg.hip): the value of a node after direction E
 // is formed from its sources' values after direction E - 1, and the thread of
-// a node's last direction stores it.  A node that no face writes is read from
+// a node's last direction stores it.  A node that no face changes is read from
 // memory: inside the block this sub-iteration's update, on a boundary plane
-// the value of the one before (floored).
+// the value of the one before (floored).  The owner of such a boundary node
+// stores it raised to the floor, which is what a reader makes of it before and
+// after that store.
 template <int E>
 struct SaBc {
     static __device__ __forceinline__ double get(const Level& L, const Fields& F, const Consts& C, const int (&p)[3],
@@ -618,7 +620,7 @@ __global__ void __launch_bounds__(256) k_sa_prep_z(ZoneGrid G) {
     const Fields F = G.z[b.z].F;
     sa_prep_body(L, F, b.bid, b.nblk);
 }
-// three waves per SIMD: fits in 168 VGPRs without spilling
+// three waves per SIMD: 168 VGPRs, two of them spilled (12 bytes per lane)
 __global__ void __launch_bounds__(kQX * kQY, 3) k_sa_rhs(Level L, Fields F, Consts C, int kc, int floored) {
     sa_rhs_body(L, F, C, kc, floored, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
                 gridDim.x * gridDim.y * gridDim.z);
