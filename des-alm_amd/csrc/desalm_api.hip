@@ -596,6 +596,7 @@ template <typename T>
 T* ws_alloc(desalm_ctx* c, long n) {
     void* p = nullptr;
     if (hipMalloc(&p, (size_t)(n > 0 ? n : 1) * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
         fail(c, "warm start: out of device memory");
         return nullptr;
     }
@@ -614,6 +615,7 @@ int ws_scratch(desalm_ctx* c, int m) {
     if (m <= w.bcap) return 0;
     const int nh = w.nh;
     MlpBuf& b = w.b;
+    w.bcap = 0;  // until every matrix is there
     b.A0 = ws_alloc<float>(c, (long)m * (kWsIn + 1));
     b.A1 = ws_alloc<float>(c, (long)m * (nh + 1));
     b.A2 = ws_alloc<float>(c, (long)m * (nh + 1));
@@ -633,6 +635,7 @@ int ws_scratch(desalm_ctx* c, int m) {
 int ws_losses(desalm_ctx* c, long n) {
     WarmStart& w = c->ws;
     if (n <= w.lcap) return 0;
+    w.lcap = 0;
     w.loss = ws_alloc<double>(c, n);
     if (!w.loss) return -1;
     w.lcap = n;
